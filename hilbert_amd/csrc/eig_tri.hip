@@ -22,7 +22,9 @@
 #include <cstdint>
 
 #include "common.hpp"
+#include "jacobi.hpp"
 #include "kernels.hpp"
+#include "refine.hpp"
 
 namespace v2h {
 
@@ -1069,6 +1071,108 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
     }
 }
 
+// Blocks of up to 16 rows: parallel cyclic Jacobi in LDS, one wavefront per
+// block.  The eigenvectors are accumulated beside the rotations (128 elements
+// per round over 64 lanes) and U+ = V diag(max(L, 0)) V^T formed from them,
+// which replaces a replay of every round; they seed the refinement of the next
+// outer iteration (vvalid; nullptr: every block is projected here).
+__device__ void project_jacobi16(const BatchDev& B, const ProjItem& it, double* work, int max_sweeps, int* vvalid) {
+    constexpr int NT = 64, DM = 16;
+    __shared__ double A[DM * (DM + 1) / 2], V[DM][DM + 1], rc[DM / 2], rs[DM / 2], red[1];
+    __shared__ int pp[DM / 2], qq[DM / 2];
+    InstState& st = B.st[it.inst];
+    const InstDev I = B.inst[it.inst];
+    const int d = it.d, dp = d + (d & 1), m = dp >> 1, t = threadIdx.x;
+    const int np = dp * (dp + 1) / 2;
+    const double mu = st.mu;
+    const double* U = B.u + I.poff + it.off;
+
+    // symmetrised upper triangle, padded to even size with a zero row
+    double nrm = 0.0;
+    for (int e = t; e < dp * dp; e += NT) {
+        const int i = e / dp, j = e - i * dp;
+        V[i][j] = i == j ? 1.0 : 0.0;
+        if (i > j) continue;
+        const double v = (j < d) ? 0.5 * (U[i * d + j] + U[j * d + i]) : 0.0;
+        A[pk(i, j)] = v;
+        nrm += (i == j ? 1.0 : 2.0) * v * v;
+    }
+    nrm = block_sum<NT>(nrm, red);
+    const double thr = 1e-30 * nrm;  // (1e-15 ||A||_F)^2
+    int nsweep = 0;
+    for (; nsweep < max_sweeps; nsweep++) {
+        double off = 0.0;
+        for (int e = t; e < dp * dp; e += NT) {
+            const int i = e / dp, j = e - i * dp;
+            if (i < j) off += 2.0 * A[pk(i, j)] * A[pk(i, j)];
+        }
+        off = block_sum<NT>(off, red);
+        if (off <= thr) break;
+        for (int r = 0; r < dp - 1; r++) {
+            if (t < m) {
+                int p, q;
+                round_pair(r, t, dp, p, q);
+                pp[t] = p;
+                qq[t] = q;
+                const double apq = A[pk(p, q)];
+                double c = 1.0, s = 0.0;
+                if (apq != 0.0) {
+                    const double th = (A[pk(q, q)] - A[pk(p, p)]) / (2.0 * apq);
+                    const double tn = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
+                    c = 1.0 / sqrt(tn * tn + 1.0);
+                    s = tn * c;
+                }
+                rc[t] = c;
+                rs[t] = s;
+            }
+            lds_sync();
+            apply_round<NT>(A, pp, qq, rc, rs, m, 1.0, true);
+            for (int e = t; e < m * dp; e += NT) {  // columns p, q of V
+                const int k = e / dp, i = e - k * dp;
+                const double c = rc[k], s = rs[k], vp = V[i][pp[k]], vq = V[i][qq[k]];
+                V[i][pp[k]] = c * vp - s * vq;
+                V[i][qq[k]] = s * vp + c * vq;
+            }
+            lds_sync();
+        }
+    }
+    if (nsweep == max_sweeps && t == 0) atomicOr(&st.status, (int)kStatusJacobiNotConverged);
+
+    // x = U+ / mu, z = U+ - sym(U), v1 = c - z; partial c.x and dual residual
+    double ex = 0.0, dr = 0.0;
+    double* X = B.x + I.poff + it.off;
+    double* Z = B.z + I.poff + it.off;
+    double* V1 = B.v1 + I.poff + it.off;
+    const double* Cc = B.c + I.poff + it.off;
+    double* Vout = work + it.work_off;
+    const double inv_mu = 1.0 / mu;
+    for (int e = t; e < d * d; e += NT) {
+        const int i = e / d, j = e - i * d;
+        double up = 0.0;
+        for (int k = 0; k < dp; k++) up += V[i][k] * (fmax(A[pk(k, k)], 0.0) * V[j][k]);
+        const double uij = U[e];
+        const double xn = up * inv_mu;
+        const double zn = up - 0.5 * (uij + U[j * d + i]);
+        const double res = (uij - mu * X[e]) + zn;
+        X[e] = xn;
+        Z[e] = zn;
+        const double ce = Cc[e];
+        V1[e] = ce - zn;
+        ex += ce * xn;
+        dr += res * res;
+        // with an odd size the zero row stays decoupled: eigenvector d is e_d
+        Vout[e] = V[i][j];
+    }
+    ex = block_sum<NT>(ex, red);
+    dr = block_sum<NT>(dr, red);
+    if (t == 0) {
+        st.pending = 1;
+        B.proj_part[2 * (size_t)it.gblock] = ex;
+        B.proj_part[2 * (size_t)it.gblock + 1] = dr;
+        if (vvalid) vvalid[it.ref] = 1;
+    }
+}
+
 // ---- One wavefront per block (blocks of up to 64 rows).  Lane j holds column
 // j of the block in registers, so the products of the Householder reduction
 // and of the back-transform are lane-local and the rank-2 updates need no
@@ -1077,7 +1181,14 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
 // that the current step cannot change are skipped (uniform branches).
 constexpr int kW = 64;
 
-__global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem* items, double* work, double* lamst) {
+//
+// After T = S L S^T the eigenvectors V = Q S are formed column by column (one
+// product and one update per reflector and no exchange, where transforming T+
+// from both sides takes the same two and a wavefront sum), then U+ from V;
+// they stay in the work area and seed the refinement of the next outer
+// iteration (vvalid; nullptr: every block is projected here).
+__global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem* items, double* work, double* lamst,
+                                                     int max_sweeps, int* vvalid, const int* route) {
     __shared__ double colb[kW];  // column k of the reduced matrix, rows >= k
     __shared__ double vbuf[kW], wbuf[kW];
     __shared__ double dd[kW], ee[kW], e2[kW], tau[kW], lamv[kW], xs[kW];
@@ -1087,6 +1198,8 @@ __global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem*
     const ProjItem it = items[blockIdx.x];
     InstState& st = B.st[it.inst];
     if (!st.active || !in_pgroup(B, it.inst)) return;
+    if (vvalid && route[it.gblock] == kRouteAccepted) return;
+    if (it.d <= 16) return project_jacobi16(B, it, work, max_sweeps, vvalid);
     const InstDev I = B.inst[it.inst];
     const int d = it.d;
     const int j = threadIdx.x;
@@ -1095,7 +1208,7 @@ __global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem*
     const double mu = st.mu;
     const double* U = B.u + I.poff + it.off;
     double* hv = work + it.work_off;     // d x d, row k = reflector k
-    double* Sv = hv + (size_t)d * d;     // d x d, column l = eigenvector l (unnormalised)
+    double* Sv = hv + (size_t)d * d;     // d x d, column l = eigenvector l (of T, unnormalised; then of U)
     double* fac = Sv + (size_t)d * d;    // 5 x d x d LU factors, [q][i][l]
     double* lprev = lamst + it.lam_off;  // d eigenvalues + last largest change
 
@@ -1126,7 +1239,6 @@ __global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem*
                 }
         }
     };
-    // tk (M v)_j over the rows i > lo (v in vbuf, zero elsewhere)
     // tk (M v)_j over the rows i > lo (v in vbuf, zero elsewhere)
     auto product = [&](int lo, double tk) {
         double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
@@ -1209,25 +1321,79 @@ __global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem*
     bool zero_block;
     const int ps = tri_eigen<kW>(d, dd, ee, e2, lamv, xs, red, lprev, Sv, fac, &st.status, tnorm, zero_block);
 
-    // ---------------------------------------------------------------- T+ in registers
+    // ---------------------------------------------------------------- V = Q S
+    {
+        const double inv = (!zero_block && j < d && xs[j] > 0.0) ? 1.0 / sqrt(xs[j]) : 0.0;
+#pragma unroll
+        for (int g = 0; g < kW / 8; g++) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) a[8 * g + u] = 0.0;
+            if (g < ng) {
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const int i = 8 * g + u;
+                    if (i < d && j < d) a[i] = zero_block ? (i == j ? 1.0 : 0.0) : Sv[(size_t)i * d + j] * inv;
+                }
+            }
+            row_fence();
+        }
+    }
+    if (d >= 3) {
+        double vnext = (j > d - 3 && j < d) ? hv[(size_t)(d - 3) * d + j] : 0.0;
+        for (int k = d - 3; k >= 0; k--) {
+            const double tk = tau[k];
+            const double vj = vnext;
+            __syncthreads();  // the readers of the previous vbuf are done
+            vbuf[j] = vj;
+            if (k > 0) vnext = (j > k - 1 && j < d) ? hv[(size_t)(k - 1) * d + j] : 0.0;
+            __syncthreads();
+            if (tk != 0.0) {
+                const double pj = product(k, tk);
+#pragma unroll
+                for (int g = 0; g < kW / 8; g++) {
+                    if (g < ng && 8 * g + 7 > k) {
+#pragma unroll
+                        for (int u = 0; u < 8; u++) a[8 * g + u] = fma(-vbuf[8 * g + u], pj, a[8 * g + u]);
+                    }
+                    row_fence();
+                }
+            }
+        }
+    }
+    if (j < d) {
+#pragma unroll
+        for (int g = 0; g < kW / 8; g++) {
+            if (g < ng) {
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    if (8 * g + u < d) Sv[(size_t)(8 * g + u) * d + j] = a[8 * g + u];
+            }
+            row_fence();
+        }
+    }
+
+    // ---------------------------------------------------------------- U+ in registers
+    // U+ = V L+ V^T, or sym(U) - V L- V^T, whichever set is smaller
     const bool use_pos = zero_block || (d - ps) <= ps;
     const int lb = use_pos ? ps : 0, le = use_pos ? d : ps;
     const double sgn = use_pos ? 1.0 : -1.0;
-    {
-        const double tjj = dd[jc], tj1 = (j + 1 < d) ? ee[j] : 0.0, tjm = (j > 0 && j < d) ? ee[j - 1] : 0.0;
-        const bool keep_t = !use_pos && j < d;
 #pragma unroll
-        for (int i = 0; i < kW; i++) {
-            double v = 0.0;
-            if (i == j) v = tjj;
-            else if (i == j + 1) v = tj1;
-            else if (i + 1 == j) v = tjm;
-            a[i] = (keep_t && i < d) ? v : 0.0;
+    for (int g = 0; g < kW / 8; g++) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) a[8 * g + u] = 0.0;
+        if (g < ng && !use_pos) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int i = 8 * g + u, ic = min(i, d - 1);
+                const double sv = 0.5 * (U[(size_t)ic * d + jc] + U[(size_t)jc * d + ic]);
+                a[i] = (i < d && j < d) ? sv : 0.0;
+            }
         }
+        row_fence();
     }
     if (!zero_block) {
         for (int l0 = lb; l0 < le; l0 += kStageMax) {
-            __syncthreads();
+            __syncthreads();  // also completes the stores of V
             for (int e = j; e < kStageMax * kW; e += kW) {
                 const int i = e / kStageMax, m = e - i * kStageMax;
                 stage[m][i] = (l0 + m < le && i < d) ? Sv[(size_t)i * d + l0 + m] : 0.0;
@@ -1235,7 +1401,7 @@ __global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem*
             __syncthreads();
             const int nm = (le - l0 < kStageMax) ? le - l0 : kStageMax;
             for (int m = 0; m < nm; m++) {
-                const double cj = sgn * lamv[l0 + m] / xs[l0 + m] * stage[m][j];
+                const double cj = sgn * lamv[l0 + m] * stage[m][j];
 #pragma unroll
                 for (int g = 0; g < kW / 8; g++) {
                     if (g < ng) {
@@ -1244,27 +1410,6 @@ __global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem*
                     }
                     row_fence();
                 }
-            }
-        }
-    }
-
-    // ---------------------------------------------------------------- U+ = Q T+ Q^T
-    if (d >= 3) {
-        double vnext = (j > d - 3 && j < d) ? hv[(size_t)(d - 3) * d + j] : 0.0;
-        for (int k = d - 3; k >= 0; k--) {
-            const double tk = tau[k];
-            const double vj = vnext;
-            __syncthreads();  // the readers of the previous vbuf / wbuf are done
-            vbuf[j] = vj;
-            if (k > 0) vnext = (j > k - 1 && j < d) ? hv[(size_t)(k - 1) * d + j] : 0.0;
-            __syncthreads();
-            if (tk != 0.0) {
-                const double pj = product(k, tk);
-                const double kk = 0.5 * tk * wsum(vj * pj);
-                const double wj = j < d ? fma(-kk, vj, pj) : 0.0;
-                wbuf[j] = wj;
-                __syncthreads();
-                update(-1, vj, wj);
             }
         }
     }
@@ -1310,6 +1455,7 @@ __global__ __launch_bounds__(kW) void k_project_wave(BatchDev B, const ProjItem*
         st.pending = 1;
         B.proj_part[2 * (size_t)it.gblock] = ex;
         B.proj_part[2 * (size_t)it.gblock + 1] = dr;
+        if (vvalid) vvalid[it.ref] = 1;
     }
 }
 
@@ -1326,13 +1472,17 @@ int project_tri_max_d(int cls) {
     return 0;
 }
 
+void launch_project_small(const BatchDev& B, const ProjItem* items, int nitems, double* work, double* lam,
+                          int max_sweeps, int* vvalid, const int* route, hipStream_t s) {
+    if (nitems > 0)
+        hipLaunchKernelGGL(k_project_wave, dim3(nitems), dim3(kW), 0, s, B, items, work, lam, max_sweeps, vvalid,
+                           route);
+}
+
 void launch_project_tri(int cls, const BatchDev& B, const ProjItem* items, int nitems, double* work, double* lam,
                         const int* route, int want, hipStream_t s) {
     if (nitems <= 0) return;
     switch (cls) {
-        case 0:
-            hipLaunchKernelGGL(k_project_wave, dim3(nitems), dim3(kW), 0, s, B, items, work, lam);
-            break;
         case 1:
             hipLaunchKernelGGL((k_project_tri<512, 8, 4, kTileReg>), dim3(nitems), dim3(512), 0, s, B, items, work, lam, route, want);
             break;

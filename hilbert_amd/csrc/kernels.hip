@@ -10,17 +10,18 @@
 //   then the end-of-iteration bookkeeping (errors, energies, mu, convergence,
 //   CG threshold).
 // * k_post : A^T y and U = mu x + A^T y - c.
-// * k_project<NT, GLOBAL> : PSD projection of one block per workgroup by
-//   parallel cyclic Jacobi on the packed upper triangle (in LDS, or in global
-//   memory for blocks too large for LDS); the rotations are recorded and
-//   replayed in reverse on diag(max(L,0)) to form U+ without an explicit
-//   eigenvector matrix.
+// * k_project<NT> : PSD projection of blocks above 256 rows by parallel cyclic
+//   Jacobi, one workgroup per block with the packed upper triangle in global
+//   memory; the rotations are
+//   recorded and replayed in reverse on diag(max(L,0)) to form U+ without an
+//   explicit eigenvector matrix.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <cstdint>
 
 #include "common.hpp"
+#include "jacobi.hpp"
 #include "kernels.hpp"
 
 namespace v2h {
@@ -501,39 +502,6 @@ __global__ __launch_bounds__(kWG) void k_spmv_plain(SellDev S, const int4* units
     if (row >= 0) out[row] = acc;
 }
 
-// ------------------------------------------------------------------------
-// PSD projection by parallel cyclic Jacobi (round-robin ordering).
-//
-// Packed upper triangle: element (i, j), i <= j, at j (j + 1) / 2 + i.
-__device__ __forceinline__ int pk(int i, int j) { return i <= j ? (j * (j + 1) >> 1) + i : (i * (i + 1) >> 1) + j; }
-
-// Pair k of round t for dp (even) indices: the circle method with index
-// dp - 1 fixed.  Returns p < q.
-__device__ __forceinline__ void round_pair(int t, int k, int dp, int& p, int& q) {
-    int M = dp - 1;
-    int a, b;
-    if (k == 0) {
-        a = t;
-        b = M;
-    } else {
-        a = t + k;
-        if (a >= M) a -= M;
-        b = t - k;
-        if (b < 0) b += M;
-    }
-    p = a < b ? a : b;
-    q = a < b ? b : a;
-}
-
-// Triangular tile index e -> (P, Q), P <= Q.
-__device__ __forceinline__ void tri_pair(int e, int& P, int& Q) {
-    int qq = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
-    while ((qq + 1) * (qq + 2) / 2 <= e) qq++;
-    while (qq * (qq + 1) / 2 > e) qq--;
-    Q = qq;
-    P = e - qq * (qq + 1) / 2;
-}
-
 template <int NT>
 __device__ __forceinline__ double block_sum(double v, double* red) {
     v = wave_sum(v);
@@ -546,68 +514,9 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
     return t;
 }
 
-// One round of two-sided rotations on the packed matrix A.  sgn = +1 applies
-// G_P T G_Q^T (forward), sgn = -1 applies G_P^T T G_Q (replay).  In the
-// forward direction the 2x2 diagonal tiles are set to their closed form.
+// Blocks too large for the tridiagonal classes: the packed matrix lives in
+// global memory.
 template <int NT>
-__device__ void apply_round(double* A, const int* pp, const int* qq, const double* rc, const double* rs,
-                            int m, double sgn, bool forward) {
-    const int ntile = m * (m + 1) / 2;
-    for (int e = threadIdx.x; e < ntile; e += NT) {
-        int P, Q;
-        tri_pair(e, P, Q);
-        const double cP = rc[P], sP = sgn * rs[P];
-        const int p = pp[P], q = qq[P];
-        if (P == Q) {
-            const int ipp = pk(p, p), ipq = pk(p, q), iqq = pk(q, q);
-            double app = A[ipp], apq = A[ipq], aqq = A[iqq];
-            if (forward) {
-                if (rs[P] != 0.0) {
-                    double t = rs[P] / rc[P];
-                    A[ipp] = app - t * apq;
-                    A[iqq] = aqq + t * apq;
-                    A[ipq] = 0.0;
-                }
-            } else {
-                // T = G^T T' G with G = [[c, -s], [s, c]] (s already negated by sgn)
-                double r00 = cP * app - sP * apq, r01 = cP * apq - sP * aqq;
-                double r10 = sP * app + cP * apq, r11 = sP * apq + cP * aqq;
-                A[ipp] = cP * r00 - sP * r01;
-                A[ipq] = sP * r00 + cP * r01;
-                A[iqq] = sP * r10 + cP * r11;
-            }
-            continue;
-        }
-        const double cQ = rc[Q], sQ = sgn * rs[Q];
-        const int r = pp[Q], s = qq[Q];
-        const int i0 = pk(p, r), i1 = pk(p, s), i2 = pk(q, r), i3 = pk(q, s);
-        double a0 = A[i0], a1 = A[i1], a2 = A[i2], a3 = A[i3];
-        // rows (p, q) by P
-        double b0 = cP * a0 - sP * a2, b1 = cP * a1 - sP * a3;
-        double b2 = sP * a0 + cP * a2, b3 = sP * a1 + cP * a3;
-        // columns (r, s) by Q
-        A[i0] = cQ * b0 - sQ * b1;
-        A[i1] = sQ * b0 + cQ * b1;
-        A[i2] = cQ * b2 - sQ * b3;
-        A[i3] = sQ * b2 + cQ * b3;
-    }
-}
-
-// Workgroup barrier that orders LDS only: outstanding global stores (the
-// rotation records) and loads (the prefetched rotations) stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-template <bool GLOBAL>
-__device__ __forceinline__ void round_sync() {
-    if constexpr (GLOBAL) __syncthreads();
-    else lds_barrier();
-}
-
-// GLOBAL: the packed matrix lives in global memory (blocks too large for LDS).
-template <int NT, bool GLOBAL>
 __global__ __launch_bounds__(NT) void k_project(BatchDev B, const ProjItem* items, double* rec_base, int max_sweeps,
                                                 double* gmat) {
     extern __shared__ double smem[];
@@ -617,8 +526,8 @@ __global__ __launch_bounds__(NT) void k_project(BatchDev B, const ProjItem* item
     const InstDev I = B.inst[it.inst];
     const int d = it.d, dp = d + (d & 1), m = dp >> 1;
     const int np = dp * (dp + 1) / 2;
-    double* A = GLOBAL ? gmat + it.mat_off : smem;
-    double* rc = GLOBAL ? smem : A + np;
+    double* A = gmat + it.mat_off;
+    double* rc = smem;
     double* rs = rc + m;
     double* red = rs + m;
     int* pp = (int*)(red + NT / 64);
@@ -677,9 +586,9 @@ __global__ __launch_bounds__(NT) void k_project(BatchDev B, const ProjItem* item
                 rec[2 * ro] = c;
                 rec[2 * ro + 1] = s;
             }
-            round_sync<GLOBAL>();
+            __syncthreads();
             apply_round<NT>(A, pp, qq, rc, rs, m, 1.0, true);
-            round_sync<GLOBAL>();
+            __syncthreads();
         }
     }
     if (nsweep == max_sweeps && threadIdx.x == 0) atomicOr(&st.status, (int)kStatusJacobiNotConverged);
@@ -720,9 +629,9 @@ __global__ __launch_bounds__(NT) void k_project(BatchDev B, const ProjItem* item
                     ns = rec[2 * ro + 1];
                 }
             }
-            round_sync<GLOBAL>();
+            __syncthreads();
             apply_round<NT>(A, pp, qq, rc, rs, m, -1.0, false);
-            round_sync<GLOBAL>();
+            __syncthreads();
         }
     }
 
@@ -853,35 +762,13 @@ void launch_spmv_plain(const SellDev& S, const int4* units, int wg0, int nwg, co
     if (nwg > 0) hipLaunchKernelGGL(k_spmv_plain, dim3(nwg), dim3(kWG), 0, s, S, units, wg0, in, out);
 }
 
-size_t project_lds_bytes(int d, int nt, bool global_matrix) {
-    int dp = d + (d & 1), m = dp / 2;
-    size_t mat = global_matrix ? 0 : (size_t)dp * (dp + 1) / 2;
-    return sizeof(double) * (mat + 2 * (size_t)m + nt / 64) + sizeof(int) * 2 * (size_t)m;
-}
-
-void launch_project(int nt, bool global_matrix, const BatchDev& B, const ProjItem* items, int nitems, int max_d,
-                    double* rec, int max_sweeps, double* gmat, hipStream_t s) {
+void launch_project(const BatchDev& B, const ProjItem* items, int nitems, int max_d, double* rec, int max_sweeps,
+                    double* gmat, hipStream_t s) {
     if (nitems <= 0) return;
-    size_t lds = project_lds_bytes(max_d, nt, global_matrix);
-    if (global_matrix) {
-        hipLaunchKernelGGL((k_project<1024, true>), dim3(nitems), dim3(1024), lds, s, B, items, rec, max_sweeps, gmat);
-        return;
-    }
-    switch (nt) {
-        case 64:
-            hipLaunchKernelGGL((k_project<64, false>), dim3(nitems), dim3(64), lds, s, B, items, rec, max_sweeps, gmat);
-            break;
-        case 256:
-            hipLaunchKernelGGL((k_project<256, false>), dim3(nitems), dim3(256), lds, s, B, items, rec, max_sweeps, gmat);
-            break;
-        case 512:
-            hipLaunchKernelGGL((k_project<512, false>), dim3(nitems), dim3(512), lds, s, B, items, rec, max_sweeps, gmat);
-            break;
-        default:
-            hipLaunchKernelGGL((k_project<1024, false>), dim3(nitems), dim3(1024), lds, s, B, items, rec, max_sweeps,
-                               gmat);
-            break;
-    }
+    constexpr int NT = 1024;
+    const size_t m = (max_d + 1) / 2;
+    const size_t lds = sizeof(double) * (2 * m + NT / 64) + sizeof(int) * 2 * m;
+    hipLaunchKernelGGL(k_project<NT>, dim3(nitems), dim3(NT), lds, s, B, items, rec, max_sweeps, gmat);
 }
 
 static int grid_for(int64_t n) {
@@ -913,17 +800,4 @@ void launch_dot1(const double* a, const double* b, int64_t n, double* out, hipSt
     hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(256), 0, s, out);
 }
 
-}  // namespace v2h
-
-namespace v2h {
-void set_project_lds_limit(size_t bytes) {
-    V2H_HIP(hipFuncSetAttribute((const void*)k_project<64, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)bytes));
-    V2H_HIP(hipFuncSetAttribute((const void*)k_project<256, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)bytes));
-    V2H_HIP(hipFuncSetAttribute((const void*)k_project<512, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)bytes));
-    V2H_HIP(hipFuncSetAttribute((const void*)k_project<1024, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)bytes));
-}
 }  // namespace v2h

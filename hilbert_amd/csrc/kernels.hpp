@@ -16,12 +16,9 @@ void launch_post(const BatchDev& B, const UnitsDev& U, hipStream_t s);
 void launch_spmv_plain(const SellDev& S, const int4* units, int wg0, int nwg, const double* in, double* out,
                        hipStream_t s);
 
-// LDS bytes of the Jacobi projection for block size d and nt threads (the
-// packed matrix is in LDS unless global_matrix).
-size_t project_lds_bytes(int d, int nt, bool global_matrix);
-void launch_project(int nt, bool global_matrix, const BatchDev& B, const ProjItem* items, int nitems, int max_d,
-                    double* rec, int max_sweeps, double* gmat, hipStream_t s);
-void set_project_lds_limit(size_t bytes);
+// Jacobi projection of blocks above 256 rows (packed matrix in gmat).
+void launch_project(const BatchDev& B, const ProjItem* items, int nitems, int max_d, double* rec, int max_sweeps,
+                    double* gmat, hipStream_t s);
 
 // Tridiagonal projection (eig_tri.hip), classes 0..4 for blocks up to
 // 64 / 128 / 192 / 224 / 256.  work: 7 d^2 doubles per block (class 4: plus
@@ -30,6 +27,13 @@ void set_project_lds_limit(size_t bytes);
 // blocks with route[global block] == want are projected.  Each reflector's tau
 // is kept on the diagonal of the reflector matrix (row k, column k).
 int project_tri_max_d(int cls);
+// Blocks of up to 64 rows, one wavefront per block (tridiagonal class 0, Jacobi
+// up to 16 rows).  Each block's eigenvectors are left after its reflectors, at
+// work + work_off + d^2 (up to 16 rows: at work + work_off).  vvalid (may be
+// null): only the blocks whose route is not kRouteAccepted are projected, and
+// their vvalid[ref] is set.
+void launch_project_small(const BatchDev& B, const ProjItem* items, int nitems, double* work, double* lam,
+                          int max_sweeps, int* vvalid, const int* route, hipStream_t s);
 void launch_project_tri(int cls, const BatchDev& B, const ProjItem* items, int nitems, double* work, double* lam,
                         const int* route, int want, hipStream_t s);
 

@@ -10,13 +10,12 @@
 namespace v2h {
 
 namespace {
-// Projection classes by block size.  Blocks of 17..256 take the tridiagonal
-// path (one wavefront per block up to 64, register tiles up to 192,
-// registers + LDS up to 224, the tile in global memory up to 256); the smallest blocks and those above 256 take
-// parallel Jacobi (packed matrix in LDS for d <= 16, in global memory beyond
-// 256).
+// Projection classes by block size, with the eigensolver of the blocks that
+// are not refined: of 17..256 rows the tridiagonal path (one wavefront per
+// block up to 64, register tiles up to 192, registers + LDS up to 224, the
+// tile in global memory up to 256), below and above parallel Jacobi (in LDS
+// for d <= 16, packed in global memory beyond 256).
 constexpr int kGlobalClass = 6;
-constexpr size_t kLdsLimit = 160 * 1024;
 constexpr int kClassThreads[Projector::kClasses] = {64, 64, 512, 768, 1024, 1024, 1024};
 constexpr int kClassTri[Projector::kClasses] = {-1, 0, 1, 2, 3, 4, -1};
 int proj_class(int d) {
@@ -64,14 +63,15 @@ void Projector::build(const std::vector<std::vector<int>>& dims, std::vector<Ins
                 it.lam_off = lam;
                 lam += dim + 1;
                 if (refined_class(k)) ritems.push_back(Refiner::Item{i, dim, it.gblock, boff, it.work_off});
-            } else {
+            } else if (k == kGlobalClass) {
                 int dp = dim + (dim & 1);
                 it.rec_off = rec;
                 rec += (int64_t)max_sweeps_ * (dp - 1) * (dp / 2) * 2;
-                if (k == kGlobalClass) {
-                    it.mat_off = mat;
-                    mat += (int64_t)dp * (dp + 1) / 2;
-                }
+                it.mat_off = mat;
+                mat += (int64_t)dp * (dp + 1) / 2;
+            } else {
+                it.work_off = work;
+                work += (int64_t)dim * dim;
             }
             cls_[k].items.push_back(it);
             nb++;
@@ -80,24 +80,34 @@ void Projector::build(const std::vector<std::vector<int>>& dims, std::vector<Ins
     }
     lam_begin_[count] = lam;
     nblocks_ = gblock;
-    size_t lds_max = 0;
+    small_.clear();
     for (int k = 0; k < kClasses; k++) {
         auto& c = cls_[k];
         c.nt = kClassThreads[k];
-        c.global = k == kGlobalClass;
         c.tri = kClassTri[k];
         std::stable_sort(c.items.begin(), c.items.end(), [](const ProjItem& a, const ProjItem& b) { return a.d > b.d; });
         c.max_d = c.items.empty() ? 0 : c.items.front().d;
-        if (!c.items.empty() && c.tri < 0) {
-            size_t lds = project_lds_bytes(c.max_d, c.nt, c.global);
-            if (lds > kLdsLimit) throw std::invalid_argument("PSD block does not fit in LDS");
-            lds_max = std::max(lds_max, lds);
-        }
         if (!c.items.empty() && c.tri >= 0 && c.max_d > project_tri_max_d(c.tri))
             throw std::logic_error("projection class table is inconsistent");
         c.d_items.upload(c.items);
     }
-    if (lds_max > 64 * 1024) set_project_lds_limit(lds_max);
+    std::vector<ProjItem> sitems;
+    for (int k : {1, 0})
+        for (ProjItem it : cls_[k].items) {
+            it.ref = (int)small_.size();
+            RefBlock b{};
+            b.inst = it.inst;
+            b.d = it.d;
+            b.gblock = it.gblock;
+            b.off = it.off;
+            // eigenvectors: after the reflectors of a tridiagonal block
+            b.w = it.work_off + (cls_[k].tri >= 0 ? (int64_t)it.d * it.d : 0);
+            small_.push_back(b);
+            sitems.push_back(it);
+        }
+    d_small_.upload(small_);
+    d_small_items_.upload(sitems);
+    d_small_valid_.upload(std::vector<int>(std::max<size_t>(small_.size(), 1), 0));
     proj_part_.alloc(2 * (size_t)std::max(gblock, 1));
     rec_.alloc(std::max<int64_t>(rec, 1));
     gmat_.alloc(std::max<int64_t>(mat, 1));
@@ -111,17 +121,26 @@ void Projector::build(const std::vector<std::vector<int>>& dims, std::vector<Ins
 void Projector::forget(int i, hipStream_t s) {
     if (lam_begin_[i + 1] > lam_begin_[i])
         launch_fill(lam_.p + lam_begin_[i], lam_begin_[i + 1] - lam_begin_[i], std::nan(""), s);
+    launch_ref_small_forget(small_dev(), (int)small_.size(), i, s);
     refiner_.forget(i, s);
 }
 
 void Projector::launch(int k, const BatchDev& B, hipStream_t s, int route) const {
     const Class& c = cls_[k];
     if (c.items.empty()) return;
-    if (c.tri >= 0)
-        launch_project_tri(c.tri, B, c.d_items.p, (int)c.items.size(), work_.p, lam_.p,
+    const int n = (int)c.items.size();
+    if (small_class(k)) {
+        const SmallDev R = small_dev();
+        const int n1 = (int)cls_[1].items.size(), all = (int)small_.size();
+        if (refine_on_) launch_ref_small(B, R, refiner_.params(), n1, all, c.max_d, s);
+        launch_project_small(B, d_small_items_.p, all, work_.p, lam_.p, max_sweeps_, refine_on_ ? R.vvalid : nullptr,
+                             R.route, s);
+    } else if (c.tri >= 0) {
+        launch_project_tri(c.tri, B, c.d_items.p, n, work_.p, lam_.p,
                            route >= 0 && refined_class(k) && refine_on() ? refiner_.route() : nullptr, route, s);
-    else
-        launch_project(c.nt, c.global, B, c.d_items.p, (int)c.items.size(), c.max_d, rec_.p, max_sweeps_, gmat_.p, s);
+    } else {
+        launch_project(B, c.d_items.p, n, c.max_d, rec_.p, max_sweeps_, gmat_.p, s);
+    }
 }
 
 }  // namespace v2h

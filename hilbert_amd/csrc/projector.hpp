@@ -25,7 +25,9 @@ class Projector {
     void build(const std::vector<std::vector<int>>& dims, std::vector<InstDev>& inst, hipStream_t s);
     // forget instance i's eigenvalues (the warm start of the tridiagonal path)
     void forget(int i, hipStream_t s);
-    bool has(int k) const { return !cls_[k].items.empty(); }
+    // Classes 0 and 1 (up to 64 rows) share their launches: class 0 is
+    // launched with class 1 where a batch has both.
+    bool has(int k) const { return !cls_[k].items.empty() && !(k == 0 && !cls_[1].items.empty()); }
     // The launch of class k.  With the refinement on, a refined class (2..5)
     // is launched twice per outer iteration: route kRouteFallback (blocks known
     // to need the tridiagonal eigensolver when the iteration starts, alongside
@@ -34,8 +36,10 @@ class Projector {
     int64_t nblocks() const { return nblocks_; }
     double* proj_part() const { return proj_part_.p; }
 
-    // Warm-started refinement (refine.hpp) for the tridiagonal classes of
-    // 65..256 rows: on by default.
+    // Warm-started refinement (refine.hpp): on by default.  The classes of up
+    // to 64 rows refine inside launch(); the tridiagonal classes of 65..256
+    // rows by the calls below.
+    static bool small_class(int k) { return k <= 1; }
     static bool refined_class(int k) { return k >= 2 && k <= 5; }
     bool refine_on() const { return refine_on_ && !refiner_.empty(); }
     void set_refine(bool on) { refine_on_ = on; }
@@ -46,17 +50,23 @@ class Projector {
     void set_refine_params(const RefParams& p) { refiner_.set_params(p); }
     const RefParams& refine_params() const { return refiner_.params(); }
     int refine_launches() const { return refiner_.launches(); }
+    // kernel launches of launch(k)
+    int class_launches(int k) const { return small_class(k) && refine_on_ ? 2 : 1; }
 
   private:
     struct Class {
         int nt = 0, max_d = 0;
-        bool global = false;
         int tri = -1;  // tridiagonal kernel class, or -1 for Jacobi
         std::vector<ProjItem> items;
         DBuf<ProjItem> d_items;
     };
     Class cls_[kClasses];
+    SmallDev small_dev() const { return SmallDev{d_small_.p, d_small_valid_.p, refiner_.route(), work_.p}; }
     DBuf<double> proj_part_, rec_, gmat_, work_, lam_;
+    std::vector<RefBlock> small_;    // class 1, then class 0, each in the order of its items
+    DBuf<RefBlock> d_small_;
+    DBuf<ProjItem> d_small_items_;
+    DBuf<int> d_small_valid_;
     std::vector<int64_t> lam_begin_;  // [count + 1] eigenvalue-store range of each instance
     int64_t nblocks_ = 0;
     int max_sweeps_ = 24;

@@ -1,5 +1,6 @@
-// refine.hpp -- warm-started PSD projection of the blocks of 65..256 rows on
-// the FP64 matrix cores (refine.hip).
+// refine.hpp -- warm-started PSD projection on the FP64 matrix cores: blocks of
+// 65..256 rows by launches over their tiles (refine.hip), blocks of up to 64
+// rows by one launch per size class (refine_small.hip).
 //
 // Between two outer iterations of BPSDP, U = mu x + A^T y - c changes little,
 // so the eigenvectors of the previous iteration almost diagonalise the new U.
@@ -115,6 +116,22 @@ void launch_ref_final(const BatchDev& B, const RefDev& R, hipStream_t s);
 void launch_ref_form_v(const BatchDev& B, const RefDev& R, hipStream_t s);
 void launch_ref_forget(const RefDev& R, int blk_begin, int blk_end, hipStream_t s);
 
+// Blocks of up to 64 rows (refine_small.hip): one launch does the whole
+// refinement; the blocks that it does not accept keep a route other than
+// kRouteAccepted and are projected by an eigensolver right after it
+// (launch_project_small), which leaves their eigenvectors in the work area and
+// sets vvalid.  There is no backoff: a failed attempt costs little.
+struct SmallDev {
+    const RefBlock* blk;  // blocks of 17..64 rows, then those of up to 16; w: the eigenvectors (d x d) in `work`
+    int* vvalid;
+    int* route;
+    double* work;
+};
+// n1 blocks of 17..64 rows, n in all, the largest of max_d rows
+void launch_ref_small(const BatchDev& B, const SmallDev& R, const RefParams& P, int n1, int n, int max_d,
+                      hipStream_t s);
+void launch_ref_small_forget(const SmallDev& R, int n, int inst, hipStream_t s);
+
 class Refiner {
   public:
     // items of the tridiagonal classes that take the refined path
@@ -134,7 +151,7 @@ class Refiner {
     // After the fallback: eigenvectors of the blocks it projected.
     void seed(const BatchDev& B, hipStream_t s) const;
     void forget(int inst, hipStream_t s) const;
-    const int* route() const { return route_.p; }
+    int* route() const { return route_.p; }
     // [block projections by the refinement, by the fallback, rejections for
     // divergence, for the correction size, for coupled clusters]
     static constexpr int kStats = 6;

@@ -987,7 +987,7 @@ void Batch::launch_projection(const BatchDev& B, bool seed, int g) {
         tstart(4 + k, ps);
         proj_.launch(k, B, ps);
         tstop(4 + k, ps);
-        launches_++;
+        launches_ += proj_.class_launches(k);
     }
     if (refine) {
         for (int pass = 0; pass < 2; pass++) {  // fallback known at the start, then the rejections

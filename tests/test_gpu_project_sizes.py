@@ -1,0 +1,85 @@
+"""GPU: the PSD projection of single blocks against LAPACK, at the sizes where
+its kernels change (16-row tiles, size classes) and for the spectra that decide
+between refinement and eigensolver.
+
+The caller-map solver with a zero map projects U = mu x - c, so a sequence of
+U is projected with whatever eigenvectors the call before left: a first block
+without any, then steps small enough to refine, then one too large.
+
+Bound: U+ is Lipschitz in U with constant 1, so a backward-stable projection is
+within a small multiple of d eps max|l| of the exact one; eps d 100 (1.4e-12 at
+d = 64) leaves room for the eigensolver's clusters, whose vectors are
+orthogonal to about 1e-5 / gap eps.
+"""
+import numpy as np
+import pytest
+
+from hilbert_amd.batch import options
+from hilbert_amd.sdp import BPSDPSolver
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(float).eps
+
+
+def _positive_part(U):
+    w, V = np.linalg.eigh(U)
+    return (V * np.maximum(w, 0.0)) @ V.T
+
+
+def _spectrum(kind, d, rng):
+    w = rng.uniform(-1.0, 1.0, d)
+    if kind == "degenerate":            # repeated eigenvalues on both sides of zero
+        w = np.round(w * 2.0) / 2.0 + 0.25
+    elif kind == "zero":                # most of the spectrum at zero
+        w[: (2 * d) // 3] = 0.0
+    elif kind == "positive":
+        w = np.abs(w) + 0.1
+    elif kind == "negative":
+        w = -np.abs(w) - 0.1
+    return w
+
+
+def _sequence(kind, d, rng):
+    """Blocks that a solve would meet one after the other."""
+    Q = np.linalg.qr(rng.standard_normal((d, d)))[0]
+    U = (Q * _spectrum(kind, d, rng)) @ Q.T
+    out = [U]
+    for step in (1e-2, 1e-3, 1e-5, 1e-9, 0.0, 1e-7):
+        G = rng.standard_normal((d, d)) / np.sqrt(d)
+        U = U + step * (G + G.T)
+        out.append(U)
+    Q = np.linalg.qr(rng.standard_normal((d, d)))[0]
+    out.append((Q * _spectrum(kind, d, rng)) @ Q.T)  # nothing in common with the one before
+    out.append(np.zeros((d, d)))
+    out.append(out[1])
+    return out
+
+
+SMALL = [1, 2, 3, 4, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64]
+
+
+@pytest.mark.parametrize("kind", ["plain", "degenerate", "zero", "positive", "negative"])
+@pytest.mark.parametrize("dims", [SMALL, [5, 16, 1], [20, 32, 7]], ids=["to64", "to16", "to32"])
+def test_projection_sequence(kind, dims):
+    rng = np.random.default_rng([len(dims), len(kind)])
+    seqs = [_sequence(kind, d, rng) for d in dims]
+    n = sum(d * d for d in dims)
+    S = BPSDPSolver(n, 1, options(e_convergence=1e-30, r_convergence=1e-30, maxiter=10 ** 6))
+    zero_a = lambda u: np.zeros(1)
+    zero_at = lambda y: np.zeros(n)
+    S.set_mu(1.0)
+    for k in range(len(seqs[0])):
+        U = [s[k] for s in seqs]
+        x = np.zeros(n)
+        c = -np.concatenate([u.ravel() for u in U])
+        S.solve(x, np.zeros(1), c, dims, 1, zero_a, zero_at)
+        mu = S.get_mu()
+        assert S.status()["status_bits"] == 0
+        off = 0
+        for d, u in zip(dims, U):
+            scale = max(np.abs(np.linalg.eigvalsh(u)).max(), 1e-300)
+            err = np.abs(mu * x[off:off + d * d].reshape(d, d) - _positive_part(u)).max() / scale
+            assert err < 100 * EPS * max(d, 10), (kind, k, d, err)
+            off += d * d
+    S.close()
