@@ -25,9 +25,23 @@ constexpr int kNT = 256;  // threads of every kernel here
 constexpr int kNB = 16;   // reflectors per compact-WY product in the eigenvector formation
 
 enum AMode : int { kAN = 0, kAT = 1, kAScaled = 2 };  // op(A)(m, k): A[m][k], A[k][m], A[m][k] s[k]
-enum BMode : int { kBN = 0, kBT = 1 };                // op(B)(k, n): B[k][n], B[n][k]
+// op(B)(k, n): B[k][n], B[n][k], or the middle factor L+ + C of U+ from S
+enum BMode : int { kBN = 0, kBT = 1, kBMiddle = 2 };
 enum Epi : int { kEpiStore = 0, kEpiAdd = 1, kEpiFinal = 2 };
-enum Gate : int { kGateRefining = 0, kGateUpdate = 1, kGateFinal = 2 };
+enum Gate : int { kGateRefining = 0, kGateUpdate = 1, kGateFinal = 2, kGateCoupled = 3 };
+constexpr int kPart = 4;  // partial values per tile
+
+// A pair too close to be separated that stays coupled by s: 0, the coupling is
+// dropped (below `keep`, or the pair's cluster is negative and has no part in
+// U+); 1, it is kept beside the eigenvalues (a positive cluster); 2, it
+// reaches across zero.  A cluster has one sign when its eigenvalues exceed the
+// row sums of the couplings, at most d max|s|.
+__device__ __forceinline__ int coupling_kind(double s, double li, double lj, double keep, int d) {
+    if (fabs(s) <= keep) return 0;
+    const double m = d * fabs(s);
+    if (fmin(li, lj) > m) return 1;
+    return fmax(li, lj) < -m ? 0 : 2;
+}
 
 // One product C = [D +] op(A) op(B) of every block, operands named by slot.
 struct Prod {
@@ -68,6 +82,25 @@ __device__ double wg_nmax(double v, double* red) {
     return t;
 }
 
+// Workgroup maxima of m[0..2] and sum f in one pass; red: 16 doubles.
+__device__ __forceinline__ void wg_tile_stats(double (&m)[3], double& f, double* red) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) m[q] = wave_nmax(m[q]);
+    f = wave_sum(f);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+        double* r = red + 4 * (threadIdx.x >> 6);
+        r[0] = m[0];
+        r[1] = m[1];
+        r[2] = m[2];
+        r[3] = f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 3; q++) m[q] = nmax(nmax(red[q], red[4 + q]), nmax(red[8 + q], red[12 + q]));
+    f = (red[3] + red[7]) + (red[11] + red[15]);
+}
+
 __device__ __forceinline__ double* slot(const RefDev& R, const RefBlock& b, int s) {
     return R.work + b.w + (int64_t)s * b.d * b.d;
 }
@@ -78,17 +111,22 @@ __device__ __forceinline__ double* lam_of(const RefDev& R, const RefBlock& b) {
 __device__ __forceinline__ bool gate_ok(const RefState& rs, int gate, int k) {
     if (gate == kGateRefining) return rs.phase == 1;
     if (gate == kGateUpdate) return rs.phase == 1 || (rs.phase == 2 && rs.cstep == k);
+    if (gate == kGateCoupled) return rs.phase == 2 && rs.coupled;
     return rs.phase == 2;
 }
 
 // ---------------------------------------------------------------- products
-// One 32 x 32 tile of one block's product.
+// One 32 x 32 tile of one block's product.  MIDDLE: the products that the
+// coupled clusters need (their own instantiation: the others keep 7 waves per
+// SIMD without it).
+template <bool MIDDLE>
 __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, const RefJob& job, const RefBlock& b,
                          const RefState& rs, double (*As)[kT + 1], double (*Bs)[kT + 1], double* red) {
     const int d = b.d;
     const int t = threadIdx.x, l = t & 63, w = t >> 6;
-    const int aslot = p.a >= 0 ? p.a : rs.xfinal;
-    const double* A = slot(R, b, aslot);
+    // the final product of a coupled block: (X (L+ + C)) X^T, the first factor in slot K
+    const bool coupled = p.epi == kEpiFinal && rs.coupled;
+    const double* A = slot(R, b, coupled ? kSlotK : (p.a >= 0 ? p.a : rs.xfinal));
     const double* Bm = slot(R, b, p.b >= 0 ? p.b : rs.xfinal);
     const double* sc = lam_of(R, b);
     const double mu = B.st[b.inst].mu;
@@ -118,7 +156,7 @@ __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, cons
             double av = 0.0;
             if (gm < d && gk < d) {
                 av = p.am == kAT ? A[(int64_t)gk * d + gm] : A[(int64_t)gm * d + gk];
-                if (p.am == kAScaled) av *= fmax(sc[gk], 0.0) * inv_mu;
+                if (p.am == kAScaled) av *= coupled ? inv_mu : fmax(sc[gk], 0.0) * inv_mu;
             }
             ra[e] = av;
             int n, kb;
@@ -131,6 +169,11 @@ __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, cons
             }
             const int gn = n0 + n, gkb = k0 + kb;
             rb[e] = (gn < d && gkb < d) ? (p.bm == kBT ? Bm[(int64_t)gn * d + gkb] : Bm[(int64_t)gkb * d + gn]) : 0.0;
+            if (MIDDLE && gn < d && gkb < d) {
+                const double lk_ = sc[gkb], ln_ = sc[gn], sv = 0.5 * (rb[e] + Bm[(int64_t)gn * d + gkb]);
+                const bool near = fabs(ln_ - lk_) <= rs.om && fabs(sv) <= rs.om;
+                rb[e] = gn == gkb ? fmax(ln_, 0.0) : (near && coupling_kind(sv, lk_, ln_, rs.keep, d) == 1 ? sv : 0.0);
+            }
         }
     };
     auto stage = [&]() {
@@ -187,6 +230,7 @@ __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, cons
     const double* U = B.u + I.poff + b.off;
     const double* Us = slot(R, b, kSlotU);
     double* V = slot(R, b, kSlotV);
+    const double* Xf = slot(R, b, rs.xfinal);
     double ex = 0.0, dr = 0.0;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -202,14 +246,14 @@ __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, cons
             V1[e] = ce - zn;
             ex += ce * xn;
             dr += res * res;
-            V[e] = A[e];
+            V[e] = Xf[e];
         }
     }
     ex = wg_sum(ex, red);
     dr = wg_sum(dr, red);
     if (t == 0) {
-        R.part[b.part + 2 * job.tile] = ex;
-        R.part[b.part + 2 * job.tile + 1] = dr;
+        R.part[b.part + kPart * job.tile] = ex;
+        R.part[b.part + kPart * job.tile + 1] = dr;
     }
 }
 
@@ -223,6 +267,7 @@ __device__ __forceinline__ int xcd_job(int bid, int n) {
     return x * per + (x < rem ? x : rem) + loc;
 }
 
+template <bool MIDDLE>
 __global__ __launch_bounds__(kNT) void k_ref_gemm(BatchDev B, RefDev R, Prod p0, Prod p1, int gate, int k) {
     __shared__ double As[kKc][kT + 1];  // As[k][m]
     __shared__ double Bs[kKc][kT + 1];  // Bs[k][n]
@@ -232,7 +277,7 @@ __global__ __launch_bounds__(kNT) void k_ref_gemm(BatchDev B, RefDev R, Prod p0,
     if (!gate_ok(rs, gate, k)) return;
     const RefBlock b = R.blk[job.blk];
     if (!in_pgroup(B, b.inst)) return;  // accepted in the other group's projection
-    ref_tile(B, R, blockIdx.y == 0 ? p0 : p1, job, b, rs, As, Bs, red);
+    ref_tile<MIDDLE>(B, R, blockIdx.y == 0 ? p0 : p1, job, b, rs, As, Bs, red);
 }
 
 // ---------------------------------------------------------------- per block
@@ -273,90 +318,138 @@ __global__ __launch_bounds__(kNT) void k_ref_sym(BatchDev B, RefDev R) {
     }
 }
 
+// The value of one tile, read by the workgroup of another tile in the same
+// launch: stored and loaded past the XCDs' L2s.
+__device__ __forceinline__ void put_part(double* p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double get_part(const double* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Corrections E of one 32 x 32 tile from S = X^T U X and G = X^T X, with the
 // eigenvalue estimates l_i = s_ii / g_ii of the block; E goes to slot K (free
-// once S is formed; G and S stay intact while other tiles read their
-// diagonals); the tile's largest correction (separated pairs) and largest
-// coupling left inside clusters go to its partial slots; diagonal tiles store
-// their l.
-__global__ __launch_bounds__(kNT) void k_ref_etile(RefDev R, RefParams P) {
-    __shared__ double li_s[32], lj_s[32];
-    __shared__ double red[4];
+// once S is formed; G and S stay intact while other tiles read them).
+//
+// The columns of X are normalised first, with n_i = g_ii^-1/2 (S and G below
+// are n_i n_j times the stored ones; X N (I + E) = X + X (N (I + E) - I)), and S
+// is symmetrised: S_ij and S_ji round differently, and that difference
+// over a narrow gap would stay in E + E^T = I - G, that is, in the
+// orthogonality of X.  The rotation part of a correction is
+// tan(th) = 2 s / (gap + sign sqrt(gap^2 + 4 s^2)), which is s / gap for
+// separated pairs and at most 1, so that a few pairs that came close since
+// the last iteration rotate by up to 45 degrees; the next step restores the
+// norms that this spoils.  Pairs within the cluster threshold (in
+// gap and coupling) keep their coupling, see coupling_kind.
+//
+// The tile's largest correction, largest coupling across zero, largest kept
+// coupling and sum of squares go to its partial values; the last tile of a
+// block to finish accepts, continues or rejects the block (step k, the updated
+// X in slot xout).
+__global__ __launch_bounds__(kNT) void k_ref_etile(RefDev R, RefParams P, int k, int xout) {
+    __shared__ double li_s[32], lj_s[32], ni_s[32], nj_s[32];
+    __shared__ double red[16];
+    __shared__ double tt[32][33];
+    __shared__ int last;
     const RefJob job = R.jobs[xcd_job(blockIdx.x, gridDim.x)];
-    if (R.rs[job.blk].phase != 1) return;
+    RefState& rs = R.rs[job.blk];
+    if (rs.phase != 1) return;
     const RefBlock b = R.blk[job.blk];
     const int d = b.d, t = threadIdx.x;
     const double* S = slot(R, b, kSlotS);
     const double* G = slot(R, b, kSlotG);
     double* E = slot(R, b, kSlotK);
+    const int i0 = job.ti * 32, j0 = job.tj * 32;
+    const int c = t & 31, r0 = t >> 5, j = j0 + c;
+    double sv4[4], gv4[4];  // rows r0 + 8 q of the tile
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int r = r0 + 8 * q, i = i0 + r, gi = j0 + r, gj = i0 + c;
+        const bool in = i < d && j < d;
+        sv4[q] = in ? S[(int64_t)i * d + j] : 0.0;
+        gv4[q] = in ? G[(int64_t)i * d + j] : 0.0;
+        tt[r][c] = (gi < d && gj < d) ? S[(int64_t)gi * d + gj] : 0.0;  // tile (tj, ti) of S
+    }
     // block scale max |l|: every tile reads the d diagonal pairs itself
     double scale = 0.0;
     for (int i = t; i < d; i += kNT) scale = nmax(scale, fabs(S[(int64_t)i * d + i] / G[(int64_t)i * d + i]));
-    scale = wg_nmax(scale, red);
-    const double om = P.cluster_rel * scale;
-    const int i0 = job.ti * 32, j0 = job.tj * 32;
-    if (t < 32) {
-        const int i = i0 + t, j = j0 + t;
-        li_s[t] = i < d ? S[(int64_t)i * d + i] / G[(int64_t)i * d + i] : 0.0;
-        lj_s[t] = j < d ? S[(int64_t)j * d + j] / G[(int64_t)j * d + j] : 0.0;
-        if (job.ti == job.tj && i < d) lam_of(R, b)[i] = li_s[t];
+    if (t < 64) {
+        const int i = (t < 32 ? i0 : j0 - 32) + t;
+        const double gd = i < d ? G[(int64_t)i * d + i] : 1.0, ld = i < d ? S[(int64_t)i * d + i] / gd : 0.0;
+        (t < 32 ? li_s : lj_s)[t & 31] = ld;
+        (t < 32 ? ni_s : nj_s)[t & 31] = 1.0 / sqrt(gd);
+        if (t < 32 && job.ti == job.tj && i < d) lam_of(R, b)[i] = ld;
     }
-    __syncthreads();
-    double me = 0.0, mc = 0.0;
-    const int c = t & 31;
-    const int j = j0 + c;
-    for (int r = t >> 5; r < 32; r += kNT / 32) {
-        const int i = i0 + r;
+    scale = wg_nmax(scale, red);
+    const double om = P.cluster_rel * scale, keep = P.accept_cpl * scale;
+    double m[3] = {0.0, 0.0, 0.0}, fr = 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int r = r0 + 8 * q, i = i0 + r;
         if (i >= d || j >= d) continue;
-        const int64_t e = (int64_t)i * d + j;
-        const double rr = (i == j ? 1.0 : 0.0) - G[e];
+        const double nn = ni_s[r] * nj_s[c], li = li_s[r], lj = lj_s[c];
         double ev;
         if (i == j) {
-            ev = 0.5 * rr;
+            ev = nj_s[c] - 1.0;
+            E[(int64_t)i * d + j] = ev;
         } else {
-            const double dl = lj_s[c] - li_s[r];
-            const double sv = S[e];
-            if (fabs(dl) > om) {
-                ev = (sv + lj_s[c] * rr) / dl;
-                me = nmax(me, fabs(ev));
+            const double rr = -gv4[q] * nn, sv = 0.5 * (sv4[q] + tt[c][r]) * nn;
+            const double dl = lj - li, sa = fma(0.5 * (lj + li), rr, sv);
+            ev = 0.5 * rr;
+            if (fabs(dl) > om || fabs(sa) > om) {
+                const double ta = sa + sa;
+                ev += ta / (dl + copysign(sqrt(fma(dl, dl, ta * ta)), dl));
             } else {
-                ev = 0.5 * rr;
-                mc = nmax(mc, fabs(sv));
+                const int kind = coupling_kind(sv, li, lj, keep, d);
+                if (kind == 1) m[2] = fmax(m[2], fabs(sv));
+                if (kind == 2) m[1] = nmax(m[1], fabs(sv));
             }
+            E[(int64_t)i * d + j] = ni_s[r] * ev;
         }
-        E[e] = ev;
+        m[0] = nmax(m[0], fabs(ev));
+        fr = fma(ev, ev, fr);
     }
-    me = wg_nmax(me, red);
-    mc = wg_nmax(mc, red);
+    wg_tile_stats(m, fr, red);
+    const int nt2 = b.nt * b.nt;
+    double* part = R.part + b.part;
     if (t == 0) {
-        R.part[b.part + 2 * job.tile] = me;
-        R.part[b.part + 2 * job.tile + 1] = scale > 0.0 ? mc / scale : mc;
+        put_part(part + kPart * job.tile, m[0]);
+        put_part(part + kPart * job.tile + 1, m[1]);
+        put_part(part + kPart * job.tile + 2, m[2]);
+        put_part(part + kPart * job.tile + 3, fr);
+        // the stores have reached memory before the ticket is drawn
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        last = __hip_atomic_fetch_add(&rs.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nt2 - 1;
     }
-}
-
-// Acceptance of step k from the tile maxima, one thread per block.
-__global__ void k_ref_decide(RefDev R, RefParams P, int k, int xout) {
-    const int bi = blockIdx.x * blockDim.x + threadIdx.x;
-    if (bi >= R.nblk) return;
-    RefState& rs = R.rs[bi];
-    if (rs.phase != 1) return;
-    const RefBlock b = R.blk[bi];
-    double me = 0.0, cpl = 0.0;
-    for (int q = 0; q < b.nt * b.nt; q++) {
-        me = nmax(me, R.part[b.part + 2 * q]);
-        cpl = nmax(cpl, R.part[b.part + 2 * q + 1]);
+    __syncthreads();
+    if (!last) return;
+    m[0] = m[1] = m[2] = fr = 0.0;
+    for (int q = t; q < nt2; q += kNT) {
+#pragma unroll
+        for (int e = 0; e < 3; e++) m[e] = nmax(m[e], get_part(part + kPart * q + e));
+        fr += get_part(part + kPart * q + 3);
     }
+    wg_tile_stats(m, fr, red);
+    if (t != 0) return;
+    const double me = m[0], mc = m[1], mk = m[2];
+    rs.ticket = 0;
+    rs.om = om;
+    rs.keep = keep;
     rs.max_e = me;
-    rs.cpl = cpl;
-    const int64_t d3 = 2 * (int64_t)b.d * b.d * b.d;
+    rs.cpl = scale > 0.0 ? mc / scale : mc;
+    const int64_t d3 = 2 * (int64_t)d * d * d;
     bool reject = false;
-    if (!(me <= 0.25) || !(cpl == cpl)) {
+    // Corrections with too large a norm do not converge.  4 + d / 10 lets a few
+    // full rotations through (a pair turned by 45 degrees adds 2) and stops a
+    // block whose eigenvectors are all new before it spends its steps.
+    if (!(fr <= 4.0 + 0.1 * d)) {
         reject = true;
         rs.rej_div += 1;
-    } else if (me <= P.accept_e && cpl <= P.accept_cpl) {
+    } else if (me <= P.accept_e && mc == 0.0) {
         rs.phase = 2;
         rs.cstep = k;
         rs.xfinal = xout;
+        rs.coupled = mk > 0.0 ? 1 : 0;
         rs.backoff = 0;
     } else if (k >= P.max_steps) {
         reject = true;
@@ -388,8 +481,8 @@ __global__ __launch_bounds__(kNT) void k_ref_close(BatchDev B, RefDev R) {
     const int nt2 = b.nt * b.nt;
     double ex = 0.0, dr = 0.0;
     for (int q = threadIdx.x; q < nt2; q += kNT) {
-        ex += R.part[b.part + 2 * q];
-        dr += R.part[b.part + 2 * q + 1];
+        ex += R.part[b.part + kPart * q];
+        dr += R.part[b.part + kPart * q + 1];
     }
     ex = wg_sum(ex, red);
     dr = wg_sum(dr, red);
@@ -399,7 +492,7 @@ __global__ __launch_bounds__(kNT) void k_ref_close(BatchDev B, RefDev R) {
         B.st[b.inst].pending = 1;
         R.route[b.gblock] = kRouteAccepted;
         rs.refined += 1;
-        rs.flops += 2 * (int64_t)b.d * b.d * b.d;
+        rs.flops += (rs.coupled ? 4 : 2) * (int64_t)b.d * b.d * b.d;
     }
 }
 
@@ -520,21 +613,23 @@ void launch_ref_step(const BatchDev& B, const RefDev& R, const RefParams& P, int
     const Prod pk{kSlotU, xin, kSlotK, -1, kAN, kBN, kEpiStore, 0};
     const Prod pg{xin, xin, kSlotG, -1, kAT, kBN, kEpiStore, 0};
     const int g = gemm_grid(R);
-    hipLaunchKernelGGL(k_ref_gemm, dim3(g, 2), dim3(kNT), 0, s, B, R, pk, pg, (int)kGateRefining, k);
+    hipLaunchKernelGGL(k_ref_gemm<false>, dim3(g, 2), dim3(kNT), 0, s, B, R, pk, pg, (int)kGateRefining, k);
     // S = X^T K
     const Prod ps{xin, kSlotK, kSlotS, -1, kAT, kBN, kEpiStore, 0};
-    hipLaunchKernelGGL(k_ref_gemm, dim3(g, 1), dim3(kNT), 0, s, B, R, ps, ps, (int)kGateRefining, k);
-    hipLaunchKernelGGL(k_ref_etile, dim3(R.njobs), dim3(kNT), 0, s, R, P);
-    hipLaunchKernelGGL(k_ref_decide, dim3((R.nblk + 255) / 256), dim3(256), 0, s, R, P, k, xout);
+    hipLaunchKernelGGL(k_ref_gemm<false>, dim3(g, 1), dim3(kNT), 0, s, B, R, ps, ps, (int)kGateRefining, k);
+    hipLaunchKernelGGL(k_ref_etile, dim3(R.njobs), dim3(kNT), 0, s, R, P, k, xout);
     // X_out = X + X E (E in slot K)
     const Prod pu{xin, kSlotK, xout, xin, kAN, kBN, kEpiAdd, 0};
-    hipLaunchKernelGGL(k_ref_gemm, dim3(g, 1), dim3(kNT), 0, s, B, R, pu, pu, (int)kGateUpdate, k);
+    hipLaunchKernelGGL(k_ref_gemm<false>, dim3(g, 1), dim3(kNT), 0, s, B, R, pu, pu, (int)kGateUpdate, k);
 }
 
 void launch_ref_final(const BatchDev& B, const RefDev& R, hipStream_t s) {
     if (R.nblk == 0) return;
+    // X (L+ + C) of the blocks with coupled clusters
+    const Prod pm{-1, kSlotS, kSlotK, -1, kAN, kBMiddle, kEpiStore, 0};
+    hipLaunchKernelGGL(k_ref_gemm<true>, dim3(gemm_grid(R), 1), dim3(kNT), 0, s, B, R, pm, pm, (int)kGateCoupled, 0);
     const Prod pf{-1, -1, -1, -1, kAScaled, kBT, kEpiFinal, 0};
-    hipLaunchKernelGGL(k_ref_gemm, dim3(gemm_grid(R), 1), dim3(kNT), 0, s, B, R, pf, pf, (int)kGateFinal, 0);
+    hipLaunchKernelGGL(k_ref_gemm<false>, dim3(gemm_grid(R), 1), dim3(kNT), 0, s, B, R, pf, pf, (int)kGateFinal, 0);
     hipLaunchKernelGGL(k_ref_close, dim3(R.nblk), dim3(kNT), 0, s, B, R);
 }
 
@@ -566,7 +661,7 @@ void Refiner::build(const std::vector<Item>& items, int count, int nblocks_total
         b.w = w;
         w += (int64_t)kRefSlots * it.d * it.d + ((it.d + 1) & ~1);
         b.part = part;
-        part += 2 * (int64_t)b.nt * b.nt;
+        part += kPart * (int64_t)b.nt * b.nt;
         for (int i = 0; i < b.nt; i++)
             for (int j = 0; j < b.nt; j++) jobs.push_back(RefJob{(int)blk_.size(), i, j, i * b.nt + j});
         blk_.push_back(b);

@@ -7,15 +7,18 @@
 // Each outer iteration refines them with the iteration of Ogita and Aishima
 // (Japan J. Indust. Appl. Math. 35, 1007 (2018)), whose steps are matrix
 // products only:
-//     G = X^T X,  S = X^T U X,  r = I - G,  l_i = s_ii / (1 - r_ii),
-//     E_ij = (s_ij + l_j r_ij) / (l_j - l_i)   (|l_j - l_i| above a cluster
-//            threshold; r_ij / 2 otherwise),    E_ii = r_ii / 2,
-//     X <- X + X E,
-// which converges quadratically, restores the orthogonality of X in the same
-// step, and then U+ = X diag(l+) X^T.  A block whose correction does not fall
-// below the acceptance threshold within max_steps steps, and every block
-// without eigenvectors yet (first iteration, after a reset), takes the
-// tridiagonal eigensolver instead; its eigenvectors seed the next iteration.
+//     G = X^T X,  S = X^T U X  (X with normalised columns),  r = I - G,
+//     l_i = s_ii,  a_ij = s_ij + (l_i + l_j) r_ij / 2,
+//     E_ij = r_ij / 2 + 2 a_ij / (l_j - l_i +- sqrt((l_j - l_i)^2 + 4 a_ij^2)),
+//     X <- X + X E
+// (the second term is their a_ij / (l_j - l_i) for small a_ij, limited like a
+// Jacobi rotation), which converges quadratically, restores the orthogonality
+// of X in the same step, and then U+ = X diag(l+) X^T.  Pairs inside a cluster
+// threshold keep only r_ij / 2 and their coupling beside diag(l+).  A block
+// whose correction does not fall below the acceptance threshold within
+// max_steps steps, and every block without eigenvectors yet (first iteration,
+// after a reset), takes the tridiagonal eigensolver instead; its eigenvectors
+// seed the next iteration.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -51,8 +54,13 @@ struct RefState {
     int phase;      // 0 idle, 1 refining, 2 accepted (at step cstep), 3 rejected
     int cstep;      // step whose correction was accepted
     int xfinal;     // slot of the accepted X
-    double max_e;   // largest correction of the last step (separated pairs)
-    double cpl;     // largest coupling left inside clusters, relative
+    double max_e;   // largest correction of the last step
+    double cpl;     // largest coupling of a cluster across zero, relative
+    // accepted with coupled clusters: pairs within om in gap and coupling whose
+    // coupling is above keep stay coupled in U+ = X (L+ + C) X^T
+    double om, keep;
+    int coupled;
+    int ticket;     // tiles of the block that finished the current step
     int64_t refined, fallback;  // counts of outer iterations on each path
     // rejections: diverging or non-finite corrections, correction above the
     // acceptance threshold after the last step, clusters left coupled
@@ -96,11 +104,14 @@ enum Route : int { kRouteFallback = 0, kRouteRefining = 1, kRouteRejected = 2, k
 struct RefParams {
     double cluster_rel = 1e-8;   // |l_i - l_j| <= cluster_rel max|l|: one cluster
     double accept_e = 2e-7;      // accept a step whose largest correction is below this
-    double accept_cpl = 1e-13;   // ... and whose clusters are decoupled to this (relative to max|l|)
-    // refinement steps before a block is rejected (1..kMaxSteps): 5 keeps
+    double accept_cpl = 1e-13;   // ... and whose clusters across zero are decoupled to this (relative to max|l|)
+    // refinement steps before a block is rejected (1..kMaxSteps): 7 keeps
     // most blocks that converge slowly off the tridiagonal fallback, whose
     // launch after the refinement is on the critical path of the iteration
-    int max_steps = 5;
+    // (8 (6e,6o) SDPs with T2: 3.02 / 2.05 / 1.55 / 1.37 ms per outer iteration
+    // with 5 / 6 / 7 / 8 steps; a step that finds nothing to do costs 7 us,
+    // 1 % of a (16e,16o) iteration)
+    int max_steps = 7;
 };
 constexpr int kMaxSteps = 8;
 
@@ -146,8 +157,8 @@ class Refiner {
     // the refinement and routes its rejections to kRouteRejected.
     void begin(const BatchDev& B, hipStream_t s) const;
     void refine(const BatchDev& B, hipStream_t s) const;
-    // kernel launches of begin() + refine(): state, sym, five per step, final product and close
-    int launches() const { return 4 + 5 * params_.max_steps; }
+    // kernel launches of begin() + refine(): state, sym, four per step, middle factor, final product and close
+    int launches() const { return 5 + 4 * params_.max_steps; }
     // After the fallback: eigenvectors of the blocks it projected.
     void seed(const BatchDev& B, hipStream_t s) const;
     void forget(int inst, hipStream_t s) const;

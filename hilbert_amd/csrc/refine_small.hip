@@ -59,10 +59,11 @@ __device__ __forceinline__ void team_sync() {
 }
 
 // One block of d <= 16 NTILE rows.  UK, X: 16 NTILE rows of stride 16 NTILE + 4;
-// lam: 16 NTILE; red: 4 per wavefront.
+// lam, nrm: 16 NTILE; red: 4 per wavefront.
 template <int NTILE, int NTHR>
 __device__ __forceinline__ void ref_small(const BatchDev& B, const SmallDev& R, const RefParams& P, const RefBlock& b,
-                                          double* UK, double* X, double* lam, double* red, int t) {
+                                          double* UK, double* X, double* lam, double* nrm, double* red,
+                                          int t) {
     constexpr int DP = 16 * NTILE, LD = DP + 4, NW = NTHR / 64;
     static_assert(NTILE <= NW, "one wavefront per 16 rows");
     const int d = b.d, l = t & 63, w = t >> 6, li = l & 15, lk = l >> 4;
@@ -131,7 +132,10 @@ __device__ __forceinline__ void ref_small(const BatchDev& B, const SmallDev& R, 
             for (int c = 0; c < NTILE; c++)
 #pragma unroll
                 for (int r = 0; r < 4; r++)
-                    if (c == w && 4 * r + lk == li) lam[m0 + li] = m0 + li < d ? s[c][r] / g[c][r] : 0.0;
+                    if (c == w && 4 * r + lk == li) {
+                        lam[m0 + li] = m0 + li < d ? s[c][r] / g[c][r] : 0.0;
+                        nrm[m0 + li] = m0 + li < d ? 1.0 / sqrt(g[c][r]) : 1.0;
+                    }
         }
         team_sync<NTHR>();  // lam; every wavefront is done with K
         if (live)
@@ -156,36 +160,39 @@ __device__ __forceinline__ void ref_small(const BatchDev& B, const SmallDev& R, 
 #pragma unroll
             for (int c = 0; c < NTILE; c++) {
                 const int j = 16 * c + li;
-                const double lj = lam[j];
+                const double lj = lam[j], nj = nrm[j];
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int i = m0 + 4 * r + lk;
-                    double ev = 0.0;
+                    double ev = 0.0, ei = 0.0, mid = 0.0;  // correction, E, middle factor
                     if (i < d && j < d) {
-                        const double rr = (i == j ? 1.0 : 0.0) - g[c][r], dl = lj - lam[i];
-                        const double sv = 0.5 * (s[c][r] + UK[j * LD + i]);
-                        const double sa = fma(0.5 * (lj + lam[i]), rr, sv);
-                        ev = 0.5 * rr;
-                        if (i != j && (fabs(dl) > om || fabs(sa) > om)) {
-                            const double ta = sa + sa;  // tan(th) = 2 sa / (dl + sign(dl) sqrt(dl^2 + 4 sa^2))
-                            ev += ta / (dl + copysign(sqrt(fma(dl, dl, ta * ta)), dl));
-                            s[c][r] = 0.0;
+                        const double ni = nrm[i], li_ = lam[i], nn = ni * nj;
+                        if (i == j) {
+                            ev = ei = nj - 1.0;
+                            mid = fmax(lj, 0.0);
                         } else {
-                            s[c][r] = i == j ? fmax(lam[i], 0.0) : 0.0;
-                            if (i != j && !(fabs(sv) <= keep)) {
-                                const double lo = fmin(lj, lam[i]), hi = fmax(lj, lam[i]);
+                            const double rr = -g[c][r] * nn, sv = 0.5 * (s[c][r] + UK[j * LD + i]) * nn;
+                            const double dl = lj - li_, sa = fma(0.5 * (lj + li_), rr, sv);
+                            ev = 0.5 * rr;
+                            if (fabs(dl) > om || fabs(sa) > om) {
+                                const double ta = sa + sa;
+                                ev += ta / (dl + copysign(sqrt(fma(dl, dl, ta * ta)), dl));
+                            } else if (!(fabs(sv) <= keep)) {
+                                const double lo = fmin(lj, li_), hi = fmax(lj, li_);
                                 if (lo > DP * fabs(sv)) {
-                                    s[c][r] = sv;
+                                    mid = sv;
                                     mk = fmax(mk, fabs(sv));
                                 } else if (!(hi < -DP * fabs(sv))) {
                                     mc = nmax(mc, fabs(sv));
                                 }
                             }
+                            ei = ni * ev;
                         }
                         fr = fma(ev, ev, fr);
                         me = nmax(me, fabs(ev));
                     }
-                    g[c][r] = ev;
+                    g[c][r] = ei;
+                    s[c][r] = mid;
                 }
             }
         }
@@ -359,24 +366,24 @@ __device__ __forceinline__ bool ref_small_begin(const BatchDev& B, const SmallDe
 template <int MT>
 __global__ __launch_bounds__(256, 2) void k_ref_small(BatchDev B, SmallDev R, RefParams P, int n1, int n) {
     constexpr int DP = 16 * MT, kMat = DP * (DP + 4) > 4 * 320 ? DP * (DP + 4) : 4 * 320;
-    __shared__ double UK[kMat], X[kMat], lam[64], red[16];
+    __shared__ double UK[kMat], X[kMat], lam[64], nrm[64], red[16];
     if ((int)blockIdx.x >= n1) {
         const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
         const int q = n1 + 4 * ((int)blockIdx.x - n1) + w;
         if (q >= n) return;
         const RefBlock b = R.blk[q];
         if (!ref_small_begin(B, R, b, R.vvalid[q], t)) return;
-        return ref_small<1, 64>(B, R, P, b, UK + w * 320, X + w * 320, lam + w * 16, nullptr, t);
+        return ref_small<1, 64>(B, R, P, b, UK + w * 320, X + w * 320, lam + w * 16, nrm + w * 16, nullptr, t);
     }
     if constexpr (MT > 1) {
         const int bi = blockIdx.x, t = threadIdx.x;
         const RefBlock b = R.blk[bi];
         if (!ref_small_begin(B, R, b, R.vvalid[bi], t)) return;
         if constexpr (MT >= 4)
-            if (b.d > 48) return ref_small<4, 256>(B, R, P, b, UK, X, lam, red, t);
+            if (b.d > 48) return ref_small<4, 256>(B, R, P, b, UK, X, lam, nrm, red, t);
         if constexpr (MT >= 3)
-            if (b.d > 32) return ref_small<3, 256>(B, R, P, b, UK, X, lam, red, t);
-        ref_small<2, 256>(B, R, P, b, UK, X, lam, red, t);
+            if (b.d > 32) return ref_small<3, 256>(B, R, P, b, UK, X, lam, nrm, red, t);
+        ref_small<2, 256>(B, R, P, b, UK, X, lam, nrm, red, t);
     }
 }
 

@@ -362,7 +362,7 @@ int v2h_batch_projection_stats(v2h_batch *b, int64_t *stats);
  * x max|l| form a cluster (default 1e-8); a step is accepted when its largest
  * correction is at most accept_e (2e-7) and the couplings left inside
  * clusters at most accept_cpl x max|l| (1e-13); a block not accepted after
- * max_steps steps (1..8, default 5) takes the tridiagonal fallback. */
+ * max_steps steps (1..8, a batch starts with 7) takes the tridiagonal fallback. */
 int v2h_batch_set_refine_params(v2h_batch *b, double cluster_rel, double accept_e, double accept_cpl,
                                 int max_steps);
 
