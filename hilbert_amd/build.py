@@ -17,7 +17,7 @@ LIB = os.path.join(HERE, "libv2rdm_hip.so")
 SOURCES = ["layout.cpp", "constraints.cpp", "sell.cpp", "rdm.cpp", "projector.cpp", "solver.cpp", "sdp_host.cpp",
            "fcidump.cpp", "writers.cpp", "orbopt_driver.cpp", "abi.cpp",
            "kernels.hip",
-           "eig_tri.hip", "refine.hip", "refine_small.hip",
+           "eig_tri.hip", "eig_big.hip", "refine.hip", "refine_small.hip",
            "df.hip", "orbopt.hip", "noalloc.hip"]
 ARCH = os.environ.get("V2H_OFFLOAD_ARCH", "gfx950")
 

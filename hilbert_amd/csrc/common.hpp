@@ -152,10 +152,7 @@ struct ProjItem {
     int inst, d, gblock;
     int ref;                // blocks of up to 64 rows: index in SmallDev (refine.hpp)
     int64_t off;            // primal offset inside the instance
-    int64_t rec_off;        // offset of the rotation record (doubles)
-    int64_t mat_off;        // offset of the packed matrix when it lives in global memory
-    int64_t work_off;       // offset of the block's work area: tridiagonal path 7 d^2 doubles, up to 16 rows
-                            // the d^2 eigenvectors
+    int64_t work_off;       // offset of the block's work area: 7 d^2 doubles, up to 16 rows the d^2 eigenvectors
     int64_t lam_off;        // tridiagonal path: offset of the block's eigenvalues (d + 1 doubles)
 };
 

@@ -25,19 +25,13 @@
 #include "jacobi.hpp"
 #include "kernels.hpp"
 #include "refine.hpp"
+#include "tri_eigen.hpp"
 
 namespace v2h {
 
 namespace {
 
-constexpr double kEps = DBL_EPSILON;
-// Consecutive eigenvalues closer than kClusterRel |lambda| + kClusterAbs ||T||
-// share a cluster; its eigenvectors are orthogonalised against each other.
-constexpr double kClusterRel = 1e-5;
-constexpr double kClusterAbs = 1e-11;
 constexpr int kStageMax = 16;    // eigenvectors per LDS chunk when forming T+
-constexpr int kMaxPasses = 160;  // Sturm passes per eigenvalue (bisection needs about 60)
-constexpr int kChunk = 8;        // inverse-iteration loads issued ahead of their use
 
 __device__ __forceinline__ void lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -173,174 +167,11 @@ __device__ __forceinline__ double reduce_scatter8(double (&v)[8]) {
     return v[0];
 }
 
-// 1/q to about 1 ulp: hardware reciprocal and one Newton step.
-__device__ __forceinline__ double recip(double q) {
-    const double r = __builtin_amdgcn_rcp(q);
-    const double e = fma(-q, r, 1.0);
-    return fma(r, e, r);
-}
-
-// Deterministic start vectors for inverse iteration, uniform in [-1, 1).
-__device__ __forceinline__ double start_value(uint32_t l, uint32_t i) {
-    uint32_t h = (l * 0x9E3779B1u) ^ ((i + 0x7F4A7C15u) * 0x85EBCA77u);
-    h ^= h >> 15;
-    h *= 0x2C1B3C6Du;
-    h ^= h >> 12;
-    h *= 0x297A2D39u;
-    h ^= h >> 15;
-    return (double)(h & 0xFFFFFFu) * (1.0 / 8388608.0) - 1.0;
-}
-
-// Sturm count of T - s I (eigenvalues below s) and S = d/ds log|det(T - s I)|
-// = sum_j 1 / (s - lambda_j), from the pivots q_i of the LDL^T recurrence.
-__device__ int sturm(double s, int d, const double* dd, const double* e2, double pivmin, double& S) {
-    double q = dd[0] - s;
-    if (fabs(q) < pivmin) q = -pivmin;
-    double r = recip(q);
-    int c = q < 0.0;
-    double dq = -1.0;
-    double acc = dq * r;
-    auto step = [&](double di, double e) {
-        double qn = fma(-e, r, di - s);
-        const double dqn = fma(e * dq, r * r, -1.0);
-        if (fabs(qn) < pivmin) qn = -pivmin;
-        r = recip(qn);
-        dq = dqn;
-        c += qn < 0.0;
-        acc = fma(dq, r, acc);
-    };
-    int i = 1;
-    for (; i + 4 <= d; i += 4) {  // the loads of four steps ahead of the recurrence
-        double dv[4], ev[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            dv[u] = dd[i + u];
-            ev[u] = e2[i + u - 1];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) step(dv[u], ev[u]);
-    }
-    for (; i < d; i++) step(dd[i], e2[i - 1]);
-    S = acc;
-    return c;
-}
-
-// Inverse-iteration helpers on one column x (stride d) of the work area, with
-// the LU factors of T - sg I in F (5 planes of stride d^2, same column).
-struct Column {
-    double* x;
-    double* F;
-    size_t ld, plane;  // d, d^2
-    __device__ double& X(int i) const { return x[(size_t)i * ld]; }
-    __device__ double& f(int q, int i) const { return F[q * plane + (size_t)i * ld]; }
-};
-
-// x <- L^{-1} P (scale x); loads run kChunk rows ahead of the recurrence.
-__device__ void apply_pl(const Column& c, int d, double scale) {
-    double bc = c.X(0) * scale;
-    for (int i0 = 0; i0 + 1 < d; i0 += kChunk) {
-        double xn[kChunk], f0[kChunk], sw[kChunk];
-#pragma unroll
-        for (int u = 0; u < kChunk; u++) {
-            const int i = min(i0 + u, d - 2);
-            xn[u] = c.X(i + 1);
-            f0[u] = c.f(0, i);
-            sw[u] = c.f(4, i);
-        }
-#pragma unroll
-        for (int u = 0; u < kChunk; u++) {
-            const int i = i0 + u;
-            if (i + 1 < d) {
-                const double bn = xn[u] * scale;
-                const bool s = sw[u] != 0.0;
-                c.X(i) = s ? bn : bc;
-                bc = s ? fma(-f0[u], bn, bc) : fma(-f0[u], bc, bn);
-            }
-        }
-    }
-    c.X(d - 1) = bc;
-}
-
-// x <- U^{-1} x; returns ||x||^2.
-__device__ double apply_u(const Column& c, int d) {
-    double x1 = 0.0, x2 = 0.0, s2 = 0.0;
-    for (int i0 = d - 1; i0 >= 0; i0 -= kChunk) {
-        double xb[kChunk], f1[kChunk], f2[kChunk], f3[kChunk];
-#pragma unroll
-        for (int u = 0; u < kChunk; u++) {
-            const int i = max(i0 - u, 0);
-            xb[u] = c.X(i);
-            f1[u] = c.f(1, i);
-            f2[u] = c.f(2, i);
-            f3[u] = c.f(3, i);
-        }
-#pragma unroll
-        for (int u = 0; u < kChunk; u++) {
-            const int i = i0 - u;
-            if (i >= 0) {
-                const double xi = fma(-f3[u], x2, fma(-f2[u], x1, xb[u])) * f1[u];
-                c.X(i) = xi;
-                s2 = fma(xi, xi, s2);
-                x2 = x1;
-                x1 = xi;
-            }
-        }
-    }
-    return s2;
-}
-
-// x <- x - sum_m (y_m . x / ||y_m||^2) y_m over the cluster's earlier columns
-// (twice); returns the new ||x||^2.
-__device__ double orthogonalise(const Column& c, int d, const double* Sv, int l0, int l, const double* xs) {
-    for (int pass = 0; pass < 2; pass++)
-        for (int m = l0; m < l; m++) {
-            const double* y = Sv + m;
-            double dot = 0.0;
-            for (int i0 = 0; i0 < d; i0 += kChunk) {
-                double yv[kChunk], xv[kChunk];
-#pragma unroll
-                for (int u = 0; u < kChunk; u++) {
-                    const int i = min(i0 + u, d - 1);
-                    yv[u] = y[(size_t)i * d];
-                    xv[u] = c.X(i);
-                }
-#pragma unroll
-                for (int u = 0; u < kChunk; u++)
-                    if (i0 + u < d) dot = fma(yv[u], xv[u], dot);
-            }
-            const double f = dot / xs[m];
-            for (int i0 = 0; i0 < d; i0 += kChunk) {
-                double yv[kChunk], xv[kChunk];
-#pragma unroll
-                for (int u = 0; u < kChunk; u++) {
-                    const int i = min(i0 + u, d - 1);
-                    yv[u] = y[(size_t)i * d];
-                    xv[u] = c.X(i);
-                }
-#pragma unroll
-                for (int u = 0; u < kChunk; u++)
-                    if (i0 + u < d) c.X(i0 + u) = fma(-f, yv[u], xv[u]);
-            }
-        }
-    double s2 = 0.0;
-    for (int i0 = 0; i0 < d; i0 += kChunk) {
-        double xv[kChunk];
-#pragma unroll
-        for (int u = 0; u < kChunk; u++) xv[u] = c.X(min(i0 + u, d - 1));
-#pragma unroll
-        for (int u = 0; u < kChunk; u++)
-            if (i0 + u < d) s2 = fma(xv[u], xv[u], s2);
-    }
-    return s2;
-}
-
-// The block's share of one thread: RI x CJ elements.  Three homes:
+// The block's share of one thread: RI x CJ elements.  Two homes:
 //   kTileReg   all in registers;
 //   kTileSplit the first kSplitRegs in registers, the rest in LDS laid out
-//              [slot][thread] (blocks just above the register budget);
-//   kTileGlobal in global memory laid out [wavefront][r][c][lane]: a
-//              wavefront's accesses coalesce (the largest blocks).
-constexpr int kTileReg = 0, kTileGlobal = 1, kTileSplit = 2;
+//              [slot][thread] (blocks just above the register budget).
+constexpr int kTileReg = 0, kTileSplit = 1;
 constexpr int kSplitRegs = 33;
 
 template <int NT, int RI, int CJ, int MODE>
@@ -374,15 +205,6 @@ struct Tile<NT, RI, CJ, kTileSplit> {
         return x;
     }
 };
-template <int NT, int RI, int CJ>
-struct Tile<NT, RI, CJ, kTileGlobal> {
-    double* p;
-    __device__ __forceinline__ double& at(int r, int c) {
-        return p[((size_t)(threadIdx.x >> 6) * RI * CJ + r * CJ + c) * 64 + (threadIdx.x & 63)];
-    }
-    __device__ __forceinline__ double col(int r, int ck) { return at(r, ck); }
-};
-
 // Eigen-decomposition of the tridiagonal T (diagonal dd, off-diagonal ee, in
 // LDS), one thread per eigenvalue: eigenvalues ascending in lamv (Sturm counts
 // and bracketed Newton steps, warm-started from lprev, which receives the new
@@ -423,68 +245,8 @@ __device__ __forceinline__ int tri_eigen(int d, const double* dd, const double* 
         const int l = t;
         double lam = 0.0;
         if (!zero_block) {
-            double lo = gl, hi = gu;
-            int clo = 0, chi = d;
-            int passes = 0;
-            double s = 0.5 * (lo + hi), S = 0.0;
-            bool haveS = false;
-            auto eval = [&](double x, double& Sx) {
-                const int c = sturm(x, d, dd, e2, pivmin, Sx);
-                passes++;
-                if (c <= l) {
-                    lo = x;
-                    clo = c;
-                } else {
-                    hi = x;
-                    chi = c;
-                }
-                return c;
-            };
             const double lp = lprev[l];
-            if (dprev >= 0.0 && isfinite(lp) && isfinite(dprev)) {
-                // expanding search around the previous eigenvalue of this block
-                double del = fmax(2.0 * dprev, 8.0 * abstol);
-                s = fmin(fmax(lp, lo), hi);
-                const int c0 = eval(s, S);
-                haveS = true;
-                for (int e = 0; e < 8; e++) {
-                    const double x = (c0 <= l) ? s + del : s - del;
-                    if (!(x > lo && x < hi)) break;
-                    double Sx;
-                    const int cx = eval(x, Sx);
-                    if ((c0 <= l) != (cx <= l)) break;
-                    del *= 4.0;
-                }
-            }
-            lam = 0.5 * (lo + hi);
-            double last = INFINITY;
-            while (passes < kMaxPasses) {
-                if (hi - lo <= abstol) {
-                    lam = 0.5 * (lo + hi);
-                    break;
-                }
-                double sn = 0.0;
-                bool newton = false;
-                if (clo == l && chi == l + 1 && haveS) {
-                    const double step = -1.0 / S;
-                    sn = s + step;
-                    if (fabs(step) <= 2.0 * abstol) {
-                        lam = fmin(fmax(sn, lo), hi);
-                        break;
-                    }
-                    newton = isfinite(sn) && sn > lo && sn < hi && fabs(step) <= 0.5 * last;
-                    if (newton) last = fabs(step);
-                }
-                if (!newton) {
-                    sn = 0.5 * (lo + hi);
-                    last = INFINITY;
-                }
-                s = sn;
-                eval(s, S);
-                haveS = true;
-                lam = s;
-            }
-            if (passes >= kMaxPasses) bad = true;
+            lam = tri_eigenvalue(l, d, dd, e2, gl, gu, abstol, pivmin, lp, dprev, bad);
             if (isfinite(lp)) change = fabs(lam - lp);
         }
         lamv[l] = lam;
@@ -497,79 +259,11 @@ __device__ __forceinline__ int tri_eigen(int d, const double* dd, const double* 
     // inverse iteration, one thread per cluster of close eigenvalues; the
     // vectors stay unnormalised, xs[l] = ||S(:, l)||^2
     if (!zero_block && t < d) {
-        auto linked = [&](int l) {
-            return l > 0 && (lamv[l] - lamv[l - 1]) <= kClusterRel * fmax(fabs(lamv[l]), fabs(lamv[l - 1])) +
-                                                           kClusterAbs * tnorm;
-        };
+        auto linked = [&](int l) { return tri_linked(lamv, l, tnorm); };
         if (!linked(t)) {
-            const int l0 = t;
-            int l1 = l0;
+            int l1 = t;
             while (l1 + 1 < d && linked(l1 + 1)) l1++;
-            const double ptol = kEps * tnorm;
-            double sprev = -INFINITY;
-            for (int l = l0; l <= l1; l++) {
-                double sg = lamv[l];
-                const double pert = 10.0 * kEps * fmax(fabs(sg), 1e-3 * tnorm);
-                if (l > l0 && sg <= sprev + pert) sg = sprev + pert;
-                sprev = sg;
-                const Column col{Sv + l, fac + l, (size_t)d, (size_t)d * d};
-                // T - sg I = P L U with partial pivoting ([q][i]: 0 multiplier,
-                // 1 reciprocal pivot, 2-3 superdiagonals of U, 4 interchange),
-                // fused with L^{-1} P applied to the start vector
-                double dcur = dd[0] - sg, ucur = d > 1 ? ee[0] : 0.0;
-                double bc = start_value((uint32_t)l, 0u);
-                for (int i = 0; i + 1 < d; i++) {
-                    const double sub = ee[i];
-                    double dnext = dd[i + 1] - sg;
-                    double unext = (i + 2 < d) ? ee[i + 1] : 0.0;
-                    const double bn = start_value((uint32_t)l, (uint32_t)(i + 1));
-                    double f, u0, u1, u2, sw, xi;
-                    if (fabs(dcur) >= fabs(sub)) {
-                        if (fabs(dcur) < ptol) dcur = (dcur < 0.0) ? -ptol : ptol;
-                        f = sub * recip(dcur);
-                        u0 = dcur;
-                        u1 = ucur;
-                        u2 = 0.0;
-                        sw = 0.0;
-                        dnext = fma(-f, ucur, dnext);
-                        xi = bc;
-                        bc = fma(-f, bc, bn);
-                    } else {
-                        f = dcur * recip(sub);
-                        u0 = sub;
-                        u1 = dnext;
-                        u2 = unext;
-                        sw = 1.0;
-                        dnext = fma(-f, dnext, ucur);
-                        unext = -f * unext;
-                        xi = bn;
-                        bc = fma(-f, bn, bc);
-                    }
-                    col.f(0, i) = f;
-                    col.f(1, i) = recip(u0);
-                    col.f(2, i) = u1;
-                    col.f(3, i) = u2;
-                    col.f(4, i) = sw;
-                    col.X(i) = xi;
-                    dcur = dnext;
-                    ucur = unext;
-                }
-                if (fabs(dcur) < ptol) dcur = (dcur < 0.0) ? -ptol : ptol;
-                col.f(1, d - 1) = recip(dcur);
-                col.f(2, d - 1) = 0.0;
-                col.f(3, d - 1) = 0.0;
-                col.X(d - 1) = bc;
-                double s2 = apply_u(col, d);
-                if (l > l0) s2 = orthogonalise(col, d, Sv, l0, l, xs);
-                apply_pl(col, d, 1.0 / sqrt(s2));
-                s2 = apply_u(col, d);
-                if (l > l0) s2 = orthogonalise(col, d, Sv, l0, l, xs);
-                if (!(s2 > 0.0) || !isfinite(s2)) {
-                    bad = true;
-                    s2 = INFINITY;  // drops the vector from T+
-                }
-                xs[l] = s2;
-            }
+            tri_vectors(t, l1, d, dd, ee, lamv, xs, tnorm, Sv, fac, bad);
         }
     }
     if (bad) atomicOr(status, (int)kStatusJacobiNotConverged);
@@ -587,7 +281,6 @@ template <int NT, int RI, int CJ, int MODE>
 __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev B, const ProjItem* items,
                                                                       double* work, double* lamst,
                                                                       const int* route, int want) {
-    constexpr bool GM = MODE == kTileGlobal;
     constexpr int PR = NT / 32;
     constexpr int DMAX = PR * RI;
     constexpr int kStage = MODE == kTileSplit ? 4 : kStageMax;  // LDS left for staging eigenvectors
@@ -598,7 +291,6 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
     static_assert(PR * RI == 32 * CJ, "square register tiling");
     __shared__ double colb[2][DMAX];
     __shared__ double pbuf[DMAX];
-    __shared__ double vbuf[DMAX], wbuf[DMAX];  // rank-2 update not yet applied to the tile
     __shared__ double dd[DMAX], ee[DMAX], e2[DMAX], tau[DMAX], lamv[DMAX], xs[DMAX];
     __shared__ double stage[kStage][DMAX];
     __shared__ double red[NT / 64];
@@ -623,9 +315,7 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
     double* lprev = lamst + it.lam_off;     // d eigenvalues + last largest change
 
     for (int i = t; i < 2 * DMAX; i += NT) (&colb[0][0])[i] = 0.0;
-    for (int i = t; i < DMAX; i += NT) vbuf[i] = wbuf[i] = 0.0;
     Tile<NT, RI, CJ, MODE> A;
-    if constexpr (GM) A.p = fac + 5 * (size_t)d * d;  // NT RI CJ doubles after the factors
     if constexpr (MODE == kTileSplit) A.lds = tile_lds;
 #pragma unroll
     for (int r = 0; r < RI; r++) {
@@ -641,21 +331,6 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
     }
     __syncthreads();
 
-    // column k of the register matrix (below the diagonal) to colb[buf], diagonal to dd[k]
-    auto put_col = [&](int k, int buf) {
-        if (tc == (k & 31)) {
-            const int ck = k >> 5;
-#pragma unroll
-            for (int r = 0; r < RI; r++) {
-                const int i = tr + PR * r;
-                const double v = A.col(r, ck);
-                if (i < d) {
-                    if (i > k) colb[buf][i] = v;
-                    else if (i == k) dd[k] = v;
-                }
-            }
-        }
-    };
     // pbuf[i] = tk (A v)_i for every row i < DMAX
     auto matvec = [&](const double (&vc)[CJ], double tk) {
         double s8[8];
@@ -674,29 +349,6 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
         const int rr = ((ln >> 4) & 1) * 4 + ((ln >> 3) & 1) * 2 + ((ln >> 2) & 1);  // reduce_scatter8 entry
         if ((ln & 3) == 0 && rr < RI) pbuf[tr_now() + PR * rr] = tk * ps;
     };
-    // A -= v w^T + w v^T, w = p - kk v, over rows/columns i with lo < i < d:
-    // v_i = vbuf[i] * vscale except v_one = 1; p in pbuf.
-    auto rank2 = [&](const double* vbuf, const double (&vc)[CJ], double vscale, int lo, int one, double kk) {
-        double wc[CJ];
-#pragma unroll
-        for (int c = 0; c < CJ; c++) {
-            const int j = tc + 32 * c;
-            const double pj = pbuf[j];
-            wc[c] = (j > lo && j < d) ? fma(-kk, vc[c], pj) : 0.0;
-        }
-#pragma unroll
-        for (int r = 0; r < RI; r++) {
-            const int i = tr + PR * r;
-            const double vraw = vbuf[i], pi = pbuf[i];
-            const bool in = i > lo && i < d;
-            const double vi = in ? (i == one ? 1.0 : vraw * vscale) : 0.0;
-            const double wi = in ? fma(-kk, vi, pi) : 0.0;
-#pragma unroll
-            for (int c = 0; c < CJ; c++) A.at(r, c) = fma(-wi, vc[c], fma(-vi, wc[c], A.at(r, c)));
-            row_fence();
-        }
-    };
-
     // Column k of the register matrix to colb[buf]: rows below the diagonal,
     // zero elsewhere; the diagonal to dd[k].
     // Row tests are made on the slot index r (a constant after unrolling)
@@ -753,58 +405,7 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
         return wsum(s);
     };
 
-    // One pass over the tile: apply the pending rank-2 update
-    // A -= v w^T + w v^T (v, w in vbuf / wbuf, zero where it does not apply)
-    // and accumulate A v_new; pbuf[i] = tk (A v_new)_i for every row i < DMAX.
-    auto fused = [&](const double (&vn)[CJ], double tk) {
-        double vo[CJ], wo[CJ];
-#pragma unroll
-        for (int c = 0; c < CJ; c++) {
-            vo[c] = vbuf[tc + 32 * c];
-            wo[c] = wbuf[tc + 32 * c];
-        }
-        double s8[8];
-#pragma unroll
-        for (int r = 0; r < 8; r++) {
-            double sr = 0.0;
-            if (r < RI) {
-                const int i = tr + PR * r;
-                const double vi = vbuf[i], wi = wbuf[i];
-#pragma unroll
-                for (int c = 0; c < CJ; c++) {
-                    const double a = fma(-wi, vo[c], fma(-vi, wo[c], A.at(r, c)));
-                    A.at(r, c) = a;
-                    sr = fma(a, vn[c], sr);
-                }
-            }
-            s8[r] = sr;
-            row_fence();
-        }
-        const double ps = reduce_scatter8(s8);
-        const int ln = lane_now();
-        const int rr = ((ln >> 4) & 1) * 4 + ((ln >> 3) & 1) * 2 + ((ln >> 2) & 1);
-        if ((ln & 3) == 0 && rr < RI) pbuf[tr_now() + PR * rr] = tk * ps;
-    };
-    // apply the pending update without a product
-    auto apply_pending = [&]() {
-        double vo[CJ], wo[CJ];
-#pragma unroll
-        for (int c = 0; c < CJ; c++) {
-            vo[c] = vbuf[tc + 32 * c];
-            wo[c] = wbuf[tc + 32 * c];
-        }
-#pragma unroll
-        for (int r = 0; r < RI; r++) {
-            const int i = tr + PR * r;
-            const double vi = vbuf[i], wi = wbuf[i];
-#pragma unroll
-            for (int c = 0; c < CJ; c++) A.at(r, c) = fma(-wi, vo[c], fma(-vi, wo[c], A.at(r, c)));
-            row_fence();
-        }
-    };
-
     // ---------------------------------------------------------------- U = Q T Q^T
-    if constexpr (!GM) {
     put_col_z(0, 0);
     for (int k = 0; k + 2 < d; k++) {
         lds_sync();
@@ -843,82 +444,6 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
     if (t == 0 && d >= 2) ee[d - 2] = colb[(d - 2) & 1][d - 1];
     __syncthreads();
 
-    } else {
-    // Step k reduces column k.  The rank-2 update of step k is applied to the
-    // tile during the product of step k + 1 (one pass per step); only the
-    // owners of column k + 1 apply it at once, to publish that column.
-    put_col(0, 0);
-    for (int k = 0; k + 2 < d; k++) {
-        lds_sync();  // column k, the pending update of step k - 1
-        const double* col = colb[k & 1];
-        double sg = 0.0;
-        for (int i = k + 2 + lane; i < DMAX; i += 64) sg = fma(col[i], col[i], sg);  // zero beyond d
-        sg = wsum(sg);
-        const double alpha = col[k + 1];
-        double tk = 0.0, sc = 0.0, beta = alpha;
-        if (sg != 0.0) {
-            beta = -copysign(sqrt(fma(alpha, alpha, sg)), alpha);
-            tk = (beta - alpha) / beta;
-            sc = 1.0 / (alpha - beta);
-        }
-        if (t == 0) {
-            ee[k] = beta;
-            tau[k] = tk;
-            hv[(size_t)k * d + k] = tk;  // tau of reflector k, read back when the eigenvectors are formed
-        }
-        // v_k = (0.., 1, col[k+2..] sc), zero when no reflection is needed
-        auto vk = [&](int i) {
-            const double ci = col[i];
-            return tk == 0.0 ? 0.0 : (i == k + 1 ? 1.0 : ((i > k + 1 && i < d) ? ci * sc : 0.0));
-        };
-        if (tk != 0.0)
-            for (int i = k + 1 + t; i < d; i += NT) hv[(size_t)k * d + i] = vk(i);
-        double vn[CJ];
-#pragma unroll
-        for (int c = 0; c < CJ; c++) vn[c] = vk(tc + 32 * c);
-        fused(vn, tk);
-        lds_sync();  // pbuf; every wavefront is done with the old vbuf / wbuf
-        double kk = 0.0;
-        for (int i = k + 1 + lane; i < d; i += 64) kk = fma(vk(i), pbuf[i], kk);
-        kk = 0.5 * tk * wsum(kk);
-        auto wk = [&](int i) { return (i > k && i < d) ? fma(-kk, vk(i), pbuf[i]) : 0.0; };
-        for (int i = t; i < DMAX; i += NT) {
-            vbuf[i] = vk(i);
-            wbuf[i] = wk(i);
-        }
-        // column k + 1 of the reduced matrix, from the owners' tile
-        if (tc == ((k + 1) & 31)) {
-            const int ck = (k + 1) >> 5;
-            const double vj = vk(k + 1), wj = wk(k + 1);
-#pragma unroll
-            for (int r = 0; r < RI; r++) {
-                const int i = tr + PR * r;
-                if (i > k && i < d) {
-                    const double a = fma(-wk(i), vj, fma(-vk(i), wj, A.col(r, ck)));
-                    if (i > k + 1) colb[(k + 1) & 1][i] = a;
-                    else dd[k + 1] = a;
-                }
-            }
-        }
-    }
-    __syncthreads();  // last column, pending update, reflector stores
-    if (d >= 2) {
-        // the last diagonal element, with the pending update applied
-        const int k = d - 1;
-        if (tc == (k & 31)) {
-            const int ck = k >> 5;
-#pragma unroll
-            for (int r = 0; r < RI; r++)
-                if (tr + PR * r == k) {
-                    const double v = vbuf[k], w = wbuf[k];
-                    dd[k] = fma(-w, v, fma(-v, w, A.col(r, ck)));
-                }
-        }
-        if (t == 0) ee[d - 2] = colb[(d - 2) & 1][d - 1];
-    }
-    __syncthreads();
-
-    }
     // ---------------------------------------------------------------- T = S L S^T
     double tnorm;
     bool zero_block;
@@ -971,7 +496,6 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
     }
 
     // ---------------------------------------------------------------- U+ = Q T+ Q^T
-    if constexpr (!GM) {
     if (d >= 3) {
         auto load_v = [&](int k, int buf) {
             if (t < DMAX) colb[buf][t] = (t > k && t < d) ? hv[(size_t)k * d + t] : 0.0;
@@ -995,41 +519,6 @@ __global__ __launch_bounds__(NT, kTriWavesPerEU<NT>) void k_project_tri(BatchDev
         }
     }
 
-    } else {
-    // M <- H_k M H_k for k = d-3 .. 0; as in the reduction, each step's
-    // rank-2 update is applied during the next step's product.
-    if (d >= 3) {
-        auto load_v = [&](int k, int buf) {
-            for (int i = t; i < DMAX; i += NT) colb[buf][i] = (i > k && i < d) ? hv[(size_t)k * d + i] : 0.0;
-        };
-        lds_sync();  // the tile's last readers of vbuf / wbuf are done
-        for (int i = t; i < DMAX; i += NT) vbuf[i] = wbuf[i] = 0.0;
-        load_v(d - 3, (d - 3) & 1);
-        for (int k = d - 3; k >= 0; k--) {
-            lds_sync();  // v_k, the pending update
-            const double tk = tau[k];
-            if (k > 0) load_v(k - 1, (k - 1) & 1);
-            if (tk != 0.0) {
-                const double* v = colb[k & 1];
-                double vn[CJ];
-#pragma unroll
-                for (int c = 0; c < CJ; c++) vn[c] = v[tc + 32 * c];
-                fused(vn, tk);
-                lds_sync();
-                double kk = 0.0;
-                for (int i = k + 1 + lane; i < d; i += 64) kk = fma(v[i], pbuf[i], kk);
-                kk = 0.5 * tk * wsum(kk);
-                for (int i = t; i < DMAX; i += NT) {
-                    vbuf[i] = v[i];
-                    wbuf[i] = i < d ? fma(-kk, v[i], pbuf[i]) : 0.0;
-                }
-            }
-        }
-        lds_sync();
-        apply_pending();
-    }
-
-    }
     // ---------------------------------------------------------------- BPSDP block update
     double ex = 0.0, dr = 0.0;
     double* X = B.x + I.poff + it.off;
@@ -1467,7 +956,6 @@ int project_tri_max_d(int cls) {
         case 1: return 128;
         case 2: return 192;
         case 3: return 224;
-        case 4: return 256;
     }
     return 0;
 }
@@ -1492,10 +980,6 @@ void launch_project_tri(int cls, const BatchDev& B, const ProjItem* items, int n
             break;
         case 3:
             hipLaunchKernelGGL((k_project_tri<1024, 7, 7, kTileSplit>), dim3(nitems), dim3(1024), 0, s, B, items,
-                               work, lam, route, want);
-            break;
-        case 4:
-            hipLaunchKernelGGL((k_project_tri<1024, 8, 8, kTileGlobal>), dim3(nitems), dim3(1024), 0, s, B, items,
                                work, lam, route, want);
             break;
         default:

@@ -10,18 +10,12 @@
 //   then the end-of-iteration bookkeeping (errors, energies, mu, convergence,
 //   CG threshold).
 // * k_post : A^T y and U = mu x + A^T y - c.
-// * k_project<NT> : PSD projection of blocks above 256 rows by parallel cyclic
-//   Jacobi, one workgroup per block with the packed upper triangle in global
-//   memory; the rotations are
-//   recorded and replayed in reverse on diag(max(L,0)) to form U+ without an
-//   explicit eigenvector matrix.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <cstdint>
 
 #include "common.hpp"
-#include "jacobi.hpp"
 #include "kernels.hpp"
 
 namespace v2h {
@@ -514,159 +508,6 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
     return t;
 }
 
-// Blocks too large for the tridiagonal classes: the packed matrix lives in
-// global memory.
-template <int NT>
-__global__ __launch_bounds__(NT) void k_project(BatchDev B, const ProjItem* items, double* rec_base, int max_sweeps,
-                                                double* gmat) {
-    extern __shared__ double smem[];
-    const ProjItem it = items[blockIdx.x];
-    InstState& st = B.st[it.inst];
-    if (!st.active || !in_pgroup(B, it.inst)) return;
-    const InstDev I = B.inst[it.inst];
-    const int d = it.d, dp = d + (d & 1), m = dp >> 1;
-    const int np = dp * (dp + 1) / 2;
-    double* A = gmat + it.mat_off;
-    double* rc = smem;
-    double* rs = rc + m;
-    double* red = rs + m;
-    int* pp = (int*)(red + NT / 64);
-    int* qq = pp + m;
-    const double mu = st.mu;
-    const double* U = B.u + I.poff + it.off;
-    double* rec = rec_base + it.rec_off;
-
-    // symmetrised upper triangle, padded to even size with a zero row
-    double nrm = 0.0;
-    for (int e = threadIdx.x; e < dp * dp; e += NT) {
-        int i = e / dp, j = e - i * dp;
-        if (i > j) continue;
-        double v = (j < d) ? 0.5 * (U[(size_t)i * d + j] + U[(size_t)j * d + i]) : 0.0;
-        A[pk(i, j)] = v;
-        nrm += (i == j ? 1.0 : 2.0) * v * v;
-    }
-    nrm = block_sum<NT>(nrm, red);
-    const double thr = 1e-30 * nrm;  // (1e-15 ||A||_F)^2
-
-    int nsweep = 0;
-    for (; nsweep < max_sweeps; nsweep++) {
-        double off = 0.0;
-        for (int e = threadIdx.x; e < np; e += NT) {
-            // e -> (i, j) column-packed, i < j contributes twice
-            int j = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
-            while ((j + 1) * (j + 2) / 2 <= e) j++;
-            while (j * (j + 1) / 2 > e) j--;
-            int i = e - j * (j + 1) / 2;
-            if (i != j) off += 2.0 * A[e] * A[e];
-        }
-        off = block_sum<NT>(off, red);
-        if (off <= thr) break;
-        // one pair per thread (m <= NT is guaranteed by the host)
-        const int k = threadIdx.x;
-        for (int t = 0; t < dp - 1; t++) {
-            if (k < m) {
-                int p, q;
-                round_pair(t, k, dp, p, q);
-                pp[k] = p;
-                qq[k] = q;
-                double apq = A[pk(p, q)];
-                double c = 1.0, s = 0.0;
-                if (apq != 0.0) {
-                    double app = A[pk(p, p)], aqq = A[pk(q, q)];
-                    double th = (aqq - app) / (2.0 * apq);
-                    double tn = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-                    c = 1.0 / sqrt(tn * tn + 1.0);
-                    s = tn * c;
-                }
-                rc[k] = c;
-                rs[k] = s;
-                // recorded for the replay; the LDS-only barrier below does not
-                // wait for these stores
-                size_t ro = ((size_t)nsweep * (dp - 1) + t) * m + k;
-                rec[2 * ro] = c;
-                rec[2 * ro + 1] = s;
-            }
-            __syncthreads();
-            apply_round<NT>(A, pp, qq, rc, rs, m, 1.0, true);
-            __syncthreads();
-        }
-    }
-    if (nsweep == max_sweeps && threadIdx.x == 0) atomicOr(&st.status, (int)kStatusJacobiNotConverged);
-
-    // U+ = J diag(max(L, 0)) J^T by replaying the rounds backwards
-    __syncthreads();  // also completes the rotation-record stores
-    for (int e = threadIdx.x; e < np; e += NT) {
-        int j = (int)((sqrtf(8.0f * (float)e + 1.0f) - 1.0f) * 0.5f);
-        while ((j + 1) * (j + 2) / 2 <= e) j++;
-        while (j * (j + 1) / 2 > e) j--;
-        int i = e - j * (j + 1) / 2;
-        double v = A[e];
-        A[e] = (i == j && v > 0.0) ? v : 0.0;
-    }
-    __syncthreads();
-    {
-        // round idx = sweep * (dp - 1) + t, replayed from last to first; the
-        // next round's rotation is fetched while the current one is applied
-        const int k = threadIdx.x;
-        const int nround = nsweep * (dp - 1);
-        double nc = 1.0, ns = 0.0;
-        if (nround > 0 && k < m) {
-            size_t ro = (size_t)(nround - 1) * m + k;
-            nc = rec[2 * ro];
-            ns = rec[2 * ro + 1];
-        }
-        for (int idx = nround - 1; idx >= 0; idx--) {
-            if (k < m) {
-                int p, q;
-                round_pair(idx % (dp - 1), k, dp, p, q);
-                pp[k] = p;
-                qq[k] = q;
-                rc[k] = nc;
-                rs[k] = ns;
-                if (idx > 0) {
-                    size_t ro = (size_t)(idx - 1) * m + k;
-                    nc = rec[2 * ro];
-                    ns = rec[2 * ro + 1];
-                }
-            }
-            __syncthreads();
-            apply_round<NT>(A, pp, qq, rc, rs, m, -1.0, false);
-            __syncthreads();
-        }
-    }
-
-    // x = U+ / mu, z = U+ - sym(U), v1 = c - z; partial c.x and dual residual
-    double ex = 0.0, dr = 0.0;
-    double* X = B.x + I.poff + it.off;
-    double* Z = B.z + I.poff + it.off;
-    double* V1 = B.v1 + I.poff + it.off;
-    const double* Cc = B.c + I.poff + it.off;
-    const double inv_mu = 1.0 / mu;
-    for (int e = threadIdx.x; e < d * d; e += NT) {
-        int i = e / d, j = e - i * d;
-        double up = A[pk(i, j)];
-        double uij = U[e];
-        double sym = 0.5 * (uij + U[(size_t)j * d + i]);
-        double xn = up * inv_mu;
-        double zn = up - sym;
-        double xo = X[e];
-        double res = (uij - mu * xo) + zn;
-        X[e] = xn;
-        Z[e] = zn;
-        double ce = Cc[e];
-        V1[e] = ce - zn;
-        ex += ce * xn;
-        dr += res * res;
-    }
-    ex = block_sum<NT>(ex, red);
-    dr = block_sum<NT>(dr, red);
-    if (threadIdx.x == 0) {
-        st.pending = 1;
-        B.proj_part[2 * (size_t)it.gblock] = ex;
-        B.proj_part[2 * (size_t)it.gblock + 1] = dr;
-    }
-}
-
 // ------------------------------------------------------------------------
 // small kernels
 
@@ -760,15 +601,6 @@ void launch_post(const BatchDev& B, const UnitsDev& U, hipStream_t s) {
 void launch_spmv_plain(const SellDev& S, const int4* units, int wg0, int nwg, const double* in, double* out,
                        hipStream_t s) {
     if (nwg > 0) hipLaunchKernelGGL(k_spmv_plain, dim3(nwg), dim3(kWG), 0, s, S, units, wg0, in, out);
-}
-
-void launch_project(const BatchDev& B, const ProjItem* items, int nitems, int max_d, double* rec, int max_sweeps,
-                    double* gmat, hipStream_t s) {
-    if (nitems <= 0) return;
-    constexpr int NT = 1024;
-    const size_t m = (max_d + 1) / 2;
-    const size_t lds = sizeof(double) * (2 * m + NT / 64) + sizeof(int) * 2 * m;
-    hipLaunchKernelGGL(k_project<NT>, dim3(nitems), dim3(NT), lds, s, B, items, rec, max_sweeps, gmat);
 }
 
 static int grid_for(int64_t n) {

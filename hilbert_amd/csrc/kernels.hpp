@@ -16,14 +16,9 @@ void launch_post(const BatchDev& B, const UnitsDev& U, hipStream_t s);
 void launch_spmv_plain(const SellDev& S, const int4* units, int wg0, int nwg, const double* in, double* out,
                        hipStream_t s);
 
-// Jacobi projection of blocks above 256 rows (packed matrix in gmat).
-void launch_project(const BatchDev& B, const ProjItem* items, int nitems, int max_d, double* rec, int max_sweeps,
-                    double* gmat, hipStream_t s);
-
-// Tridiagonal projection (eig_tri.hip), classes 0..4 for blocks up to
-// 64 / 128 / 192 / 224 / 256.  work: 7 d^2 doubles per block (class 4: plus
-// 1024 x 64 for the tile); lam: d + 1 doubles per block, kept between calls
-// (NaN = no previous eigenvalues).  route (may be null, classes 1-4): only
+// Tridiagonal projection (eig_tri.hip), classes 0..3 for blocks up to
+// 64 / 128 / 192 / 224.  work: 7 d^2 doubles per block; lam: d + 1 doubles per block, kept between calls
+// (NaN = no previous eigenvalues).  route (may be null, classes 1-3): only
 // blocks with route[global block] == want are projected.  Each reflector's tau
 // is kept on the diagonal of the reflector matrix (row k, column k).
 int project_tri_max_d(int cls);

@@ -11,13 +11,10 @@ namespace v2h {
 
 namespace {
 // Projection classes by block size, with the eigensolver of the blocks that
-// are not refined: of 17..256 rows the tridiagonal path (one wavefront per
-// block up to 64, register tiles up to 192, registers + LDS up to 224, the
-// tile in global memory up to 256), below and above parallel Jacobi (in LDS
-// for d <= 16, packed in global memory beyond 256).
-constexpr int kGlobalClass = 6;
-constexpr int kClassThreads[Projector::kClasses] = {64, 64, 512, 768, 1024, 1024, 1024};
-constexpr int kClassTri[Projector::kClasses] = {-1, 0, 1, 2, 3, 4, -1};
+// are not refined: Jacobi up to 16 rows, the tridiagonal path in one wavefront
+// per block up to 64, in register tiles up to 192, in registers and LDS up to
+// 224, and spread over the GPU beyond (eig_big.hip).
+constexpr int kClassTri[Projector::kClasses] = {-1, 0, 1, 2, 3, -1, -1};
 int proj_class(int d) {
     if (d <= 16) return 0;
     if (d <= 64) return 1;
@@ -25,16 +22,18 @@ int proj_class(int d) {
     if (d <= 192) return 3;
     if (d <= 224) return 4;
     if (d <= 256) return 5;
-    return kGlobalClass;
+    return 6;
 }
-// work doubles of a tridiagonal-path block: reflectors, eigenvectors, LU
-// factors (7 d^2), plus the tile of the global-memory class
-int64_t tri_work(int tri, int d) { return 7 * (int64_t)d * d + (tri == 4 ? (int64_t)1024 * 8 * 8 : 0); }
+// work doubles of a block: eigenvectors, and above 16 rows reflectors and LU
+// factors (7 d^2 in all), above 224 also a few vectors
+int64_t work_size(int k, int64_t d) {
+    return k == 0 ? d * d : 7 * d * d + (Projector::big_class(k) ? 8 * d : 0);
+}
 }  // namespace
 
 void Projector::build(const std::vector<std::vector<int>>& dims, std::vector<InstDev>& inst, hipStream_t s) {
     int gblock = 0;
-    int64_t rec = 0, mat = 0, work = 0, lam = 0;
+    int64_t work = 0, lam = 0;
     const int count = (int)dims.size();
     std::vector<Refiner::Item> ritems;
     for (auto& c : cls_) c.items.clear();
@@ -49,30 +48,19 @@ void Projector::build(const std::vector<std::vector<int>>& dims, std::vector<Ins
             off += (int64_t)dim * dim;
             if (dim == 0) continue;
             const int k = proj_class(dim);
-            // the Jacobi kernels give each rotation pair one thread
-            if (kClassTri[k] < 0 && (dim + 1) / 2 > kClassThreads[k])
-                throw std::invalid_argument("PSD block larger than 2048 is not supported");
+            if (dim > kBigMaxRows) throw std::invalid_argument("PSD block larger than 2048 is not supported");
             ProjItem it{};
             it.inst = i;
             it.d = dim;
             it.gblock = gblock++;
             it.off = boff;
+            it.work_off = work;
+            work += work_size(k, dim);
             if (kClassTri[k] >= 0) {
-                it.work_off = work;
-                work += tri_work(kClassTri[k], dim);
                 it.lam_off = lam;
                 lam += dim + 1;
-                if (refined_class(k)) ritems.push_back(Refiner::Item{i, dim, it.gblock, boff, it.work_off});
-            } else if (k == kGlobalClass) {
-                int dp = dim + (dim & 1);
-                it.rec_off = rec;
-                rec += (int64_t)max_sweeps_ * (dp - 1) * (dp / 2) * 2;
-                it.mat_off = mat;
-                mat += (int64_t)dp * (dp + 1) / 2;
-            } else {
-                it.work_off = work;
-                work += (int64_t)dim * dim;
             }
+            if (!small_class(k)) ritems.push_back(Refiner::Item{i, dim, it.gblock, boff, it.work_off});
             cls_[k].items.push_back(it);
             nb++;
         }
@@ -83,7 +71,6 @@ void Projector::build(const std::vector<std::vector<int>>& dims, std::vector<Ins
     small_.clear();
     for (int k = 0; k < kClasses; k++) {
         auto& c = cls_[k];
-        c.nt = kClassThreads[k];
         c.tri = kClassTri[k];
         std::stable_sort(c.items.begin(), c.items.end(), [](const ProjItem& a, const ProjItem& b) { return a.d > b.d; });
         c.max_d = c.items.empty() ? 0 : c.items.front().d;
@@ -109,8 +96,6 @@ void Projector::build(const std::vector<std::vector<int>>& dims, std::vector<Ins
     d_small_items_.upload(sitems);
     d_small_valid_.upload(std::vector<int>(std::max<size_t>(small_.size(), 1), 0));
     proj_part_.alloc(2 * (size_t)std::max(gblock, 1));
-    rec_.alloc(std::max<int64_t>(rec, 1));
-    gmat_.alloc(std::max<int64_t>(mat, 1));
     work_.alloc(std::max<int64_t>(work, 1));
     lam_.alloc(std::max<int64_t>(lam, 1));
     launch_fill(lam_.p, std::max<int64_t>(lam, 1), std::nan(""), s);
@@ -135,11 +120,9 @@ void Projector::launch(int k, const BatchDev& B, hipStream_t s, int route) const
         if (refine_on_) launch_ref_small(B, R, refiner_.params(), n1, all, c.max_d, s);
         launch_project_small(B, d_small_items_.p, all, work_.p, lam_.p, max_sweeps_, refine_on_ ? R.vvalid : nullptr,
                              R.route, s);
-    } else if (c.tri >= 0) {
+    } else {
         launch_project_tri(c.tri, B, c.d_items.p, n, work_.p, lam_.p,
                            route >= 0 && refined_class(k) && refine_on() ? refiner_.route() : nullptr, route, s);
-    } else {
-        launch_project(B, c.d_items.p, n, c.max_d, rec_.p, max_sweeps_, gmat_.p, s);
     }
 }
 

@@ -16,7 +16,7 @@ namespace v2h {
 
 class Projector {
   public:
-    // Jacobi d <= 16, tridiagonal d <= 64 / 128 / 192 / 224 / 256, Jacobi d > 256
+    // d <= 16 / 64 / 128 / 192 / 224 / 256, d > 256
     static constexpr int kClasses = 7;
 
     // dims[i]: PSD block sizes of instance i in primal order (zeros allowed);
@@ -27,8 +27,9 @@ class Projector {
     void forget(int i, hipStream_t s);
     // Classes 0 and 1 (up to 64 rows) share their launches: class 0 is
     // launched with class 1 where a batch has both.
-    bool has(int k) const { return !cls_[k].items.empty() && !(k == 0 && !cls_[1].items.empty()); }
-    // The launch of class k.  With the refinement on, a refined class (2..5)
+    // Classes 5 and 6 are projected by project_big.
+    bool has(int k) const { return !cls_[k].items.empty() && !big_class(k) && !(k == 0 && !cls_[1].items.empty()); }
+    // The launch of class k.  With the refinement on, a refined class (2..4)
     // is launched twice per outer iteration: route kRouteFallback (blocks known
     // to need the tridiagonal eigensolver when the iteration starts, alongside
     // the refinement) and kRouteRejected (after it); route < 0: every block.
@@ -37,10 +38,14 @@ class Projector {
     double* proj_part() const { return proj_part_.p; }
 
     // Warm-started refinement (refine.hpp): on by default.  The classes of up
-    // to 64 rows refine inside launch(); the tridiagonal classes of 65..256
-    // rows by the calls below.
+    // to 64 rows refine inside launch(); the others by the calls below.
     static bool small_class(int k) { return k <= 1; }
-    static bool refined_class(int k) { return k >= 2 && k <= 5; }
+    static bool refined_class(int k) { return k >= 2 && k <= 4; }
+    static bool big_class(int k) { return k >= 5; }
+    // Classes 5 and 6: after refine_run where the refinement is on.  Returns the
+    // kernel launches.
+    bool has_big() const { return refiner_.has_big(); }
+    int project_big(const BatchDev& B, hipStream_t s) { return refiner_.project_big(B, refine_on(), s); }
     bool refine_on() const { return refine_on_ && !refiner_.empty(); }
     void set_refine(bool on) { refine_on_ = on; }
     void refine_begin(const BatchDev& B, hipStream_t s) const { refiner_.begin(B, s); }
@@ -55,14 +60,14 @@ class Projector {
 
   private:
     struct Class {
-        int nt = 0, max_d = 0;
-        int tri = -1;  // tridiagonal kernel class, or -1 for Jacobi
+        int max_d = 0;
+        int tri = -1;  // tridiagonal kernel class of eig_tri.hip, or -1
         std::vector<ProjItem> items;
         DBuf<ProjItem> d_items;
     };
     Class cls_[kClasses];
     SmallDev small_dev() const { return SmallDev{d_small_.p, d_small_valid_.p, refiner_.route(), work_.p}; }
-    DBuf<double> proj_part_, rec_, gmat_, work_, lam_;
+    DBuf<double> proj_part_, work_, lam_;
     std::vector<RefBlock> small_;    // class 1, then class 0, each in the order of its items
     DBuf<RefBlock> d_small_;
     DBuf<ProjItem> d_small_items_;

@@ -28,7 +28,7 @@ enum AMode : int { kAN = 0, kAT = 1, kAScaled = 2 };  // op(A)(m, k): A[m][k], A
 // op(B)(k, n): B[k][n], B[n][k], or the middle factor L+ + C of U+ from S
 enum BMode : int { kBN = 0, kBT = 1, kBMiddle = 2 };
 enum Epi : int { kEpiStore = 0, kEpiAdd = 1, kEpiFinal = 2 };
-enum Gate : int { kGateRefining = 0, kGateUpdate = 1, kGateFinal = 2, kGateCoupled = 3 };
+enum Gate : int { kGateRefining = 0, kGateUpdate = 1, kGateFinal = 2, kGateCoupled = 3, kGateFresh = 4 };
 constexpr int kPart = 4;  // partial values per tile
 
 // A pair too close to be separated that stays coupled by s: 0, the coupling is
@@ -112,6 +112,7 @@ __device__ __forceinline__ bool gate_ok(const RefState& rs, int gate, int k) {
     if (gate == kGateRefining) return rs.phase == 1;
     if (gate == kGateUpdate) return rs.phase == 1 || (rs.phase == 2 && rs.cstep == k);
     if (gate == kGateCoupled) return rs.phase == 2 && rs.coupled;
+    if (gate == kGateFresh) return rs.phase == kPhaseFresh;
     return rs.phase == 2;
 }
 
@@ -246,7 +247,7 @@ __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, cons
             V1[e] = ce - zn;
             ex += ce * xn;
             dr += res * res;
-            V[e] = Xf[e];
+            if (Xf != V) V[e] = Xf[e];
         }
     }
     ex = wg_sum(ex, red);
@@ -461,21 +462,23 @@ __global__ __launch_bounds__(kNT) void k_ref_etile(RefDev R, RefParams P, int k,
     rs.flops += (reject ? 3 : 4) * d3;  // a rejected block skips X + XE
     if (reject) {
         rs.phase = 3;
-        const int bo = min(2 * rs.backoff + 2, kMaxBackoff);
+        // above kTriMaxRows the eigensolver costs many times a failed attempt
+        const int bo = d > kTriMaxRows ? 0 : min(2 * rs.backoff + 2, kMaxBackoff);
         rs.backoff = bo;
         rs.wait = bo;
         R.route[b.gblock] = kRouteRejected;
     }
 }
 
-// Block sums of the accepted blocks (tile partials in a fixed order).
-__global__ __launch_bounds__(kNT) void k_ref_close(BatchDev B, RefDev R) {
+// Block sums of the accepted blocks, or (fresh) of those whose eigenvectors
+// were just computed (tile partials in a fixed order).
+__global__ __launch_bounds__(kNT) void k_ref_close(BatchDev B, RefDev R, int fresh) {
     __shared__ double red[4];
     const RefBlock b = R.blk[blockIdx.x];
     if (!in_pgroup(B, b.inst)) return;
     RefState& rs = R.rs[blockIdx.x];
-    if (rs.phase != 2) {  // projected by the tridiagonal fallback this iteration
-        if (threadIdx.x == 0 && B.st[b.inst].active) rs.fallback += 1;
+    if (rs.phase != (fresh ? kPhaseFresh : 2)) {  // projected by the eigensolver this iteration
+        if (!fresh && threadIdx.x == 0 && B.st[b.inst].active) rs.fallback += 1;
         return;
     }
     const int nt2 = b.nt * b.nt;
@@ -490,6 +493,7 @@ __global__ __launch_bounds__(kNT) void k_ref_close(BatchDev B, RefDev R) {
         B.proj_part[2 * (size_t)b.gblock] = ex;
         B.proj_part[2 * (size_t)b.gblock + 1] = dr;
         B.st[b.inst].pending = 1;
+        if (fresh) return;
         R.route[b.gblock] = kRouteAccepted;
         rs.refined += 1;
         rs.flops += (rs.coupled ? 4 : 2) * (int64_t)b.d * b.d * b.d;
@@ -507,7 +511,7 @@ __global__ __launch_bounds__(kNT) void k_ref_form_v(BatchDev B, RefDev R) {
     __shared__ double Tm[kNB][kNB];
     __shared__ double tau[kNB];
     const RefBlock b = R.blk[blockIdx.x];
-    if (!in_pgroup(B, b.inst)) return;
+    if (!in_pgroup(B, b.inst) || b.d > kTriMaxRows) return;  // (the larger ones have theirs from eig_big.hip)
     RefState& rs = R.rs[blockIdx.x];
     // blocks that took the fallback and try the refinement next iteration
     const int route = R.route[b.gblock];
@@ -630,7 +634,13 @@ void launch_ref_final(const BatchDev& B, const RefDev& R, hipStream_t s) {
     hipLaunchKernelGGL(k_ref_gemm<true>, dim3(gemm_grid(R), 1), dim3(kNT), 0, s, B, R, pm, pm, (int)kGateCoupled, 0);
     const Prod pf{-1, -1, -1, -1, kAScaled, kBT, kEpiFinal, 0};
     hipLaunchKernelGGL(k_ref_gemm<false>, dim3(gemm_grid(R), 1), dim3(kNT), 0, s, B, R, pf, pf, (int)kGateFinal, 0);
-    hipLaunchKernelGGL(k_ref_close, dim3(R.nblk), dim3(kNT), 0, s, B, R);
+    hipLaunchKernelGGL(k_ref_close, dim3(R.nblk), dim3(kNT), 0, s, B, R, 0);
+}
+
+void launch_ref_fresh(const BatchDev& B, const RefDev& R, hipStream_t s) {
+    const Prod pf{-1, -1, -1, -1, kAScaled, kBT, kEpiFinal, 0};
+    hipLaunchKernelGGL(k_ref_gemm<false>, dim3(gemm_grid(R), 1), dim3(kNT), 0, s, B, R, pf, pf, (int)kGateFresh, 0);
+    hipLaunchKernelGGL(k_ref_close, dim3(R.nblk), dim3(kNT), 0, s, B, R, 1);
 }
 
 void launch_ref_form_v(const BatchDev& B, const RefDev& R, hipStream_t s) {
@@ -649,7 +659,7 @@ void Refiner::build(const std::vector<Item>& items, int count, int nblocks_total
     int64_t w = 0, part = 0;
     int cur = 0;
     for (const Item& it : items) {
-        if (it.d > 256) throw std::logic_error("refined projection: block larger than 256");
+        if (it.d > kBigMaxRows) throw std::logic_error("refined projection: block too large");
         while (cur < it.inst) inst_begin_[++cur] = (int)blk_.size();
         RefBlock b{};
         b.inst = it.inst;
@@ -667,6 +677,16 @@ void Refiner::build(const std::vector<Item>& items, int count, int nblocks_total
         blk_.push_back(b);
     }
     while (cur < count) inst_begin_[++cur] = (int)blk_.size();
+    big_.clear();
+    big_max_ = 0;
+    for (int i = 0; i < (int)blk_.size(); i++)
+        if (blk_[i].d > kTriMaxRows) {
+            big_.push_back(i);
+            big_max_ = std::max(big_max_, blk_[i].d);
+        }
+    d_big_.upload(big_);
+    need_.upload(std::vector<int>(big_.size(), 0));
+    need_host_.assign(big_.size(), 0);
     njobs_ = (int)jobs.size();
     d_blk_.upload(blk_);
     d_jobs_.upload(jobs);
@@ -703,6 +723,27 @@ void Refiner::refine(const BatchDev& B, hipStream_t s) const {
     launch_ref_sym(B, R, s);
     for (int k = 1; k <= params_.max_steps; k++) launch_ref_step(B, R, params_, k, s);
     launch_ref_final(B, R, s);
+}
+
+int Refiner::project_big(const BatchDev& B, bool refined, hipStream_t s) {
+    const int n = (int)big_.size();
+    if (n == 0) return 0;
+    const RefDev R = dev();
+    launch_big_need(B, R, d_big_.p, n, refined, need_.p, s);
+    int max_d = big_max_;
+    if (refined) {
+        // the eigensolver is some hundred launches, nearly always for nothing:
+        // worth a look at what is needed
+        V2H_HIP(hipMemcpyAsync(need_host_.data(), need_.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
+        V2H_HIP(hipStreamSynchronize(s));
+        max_d = 0;
+        for (int i = 0; i < n; i++)
+            if (need_host_[i]) max_d = std::max(max_d, blk_[big_[i]].d);
+        if (max_d == 0) return 1;
+    }
+    const int l = launch_big_eig(B, R, d_big_.p, need_.p, n, max_d, s);
+    launch_ref_fresh(B, R, s);
+    return l + 3;
 }
 
 void Refiner::seed(const BatchDev& B, hipStream_t s) const {

@@ -1,5 +1,5 @@
-// refine.hpp -- warm-started PSD projection on the FP64 matrix cores: blocks of
-// 65..256 rows by launches over their tiles (refine.hip), blocks of up to 64
+// refine.hpp -- warm-started PSD projection on the FP64 matrix cores: blocks
+// above 64 rows by launches over their tiles (refine.hip), blocks of up to 64
 // rows by one launch per size class (refine_small.hip).
 //
 // Between two outer iterations of BPSDP, U = mu x + A^T y - c changes little,
@@ -17,8 +17,8 @@
 // threshold keep only r_ij / 2 and their coupling beside diag(l+).  A block
 // whose correction does not fall below the acceptance threshold within
 // max_steps steps, and every block without eigenvectors yet (first iteration,
-// after a reset), takes the tridiagonal eigensolver instead; its eigenvectors
-// seed the next iteration.
+// after a reset), takes a tridiagonal eigensolver instead (eig_tri.hip, above
+// 224 rows eig_big.hip); its eigenvectors seed the next iteration.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -51,7 +51,7 @@ struct RefJob {
 // Per-block state of the refinement.
 struct RefState {
     int vvalid;     // slot V holds eigenvector estimates of a recent U
-    int phase;      // 0 idle, 1 refining, 2 accepted (at step cstep), 3 rejected
+    int phase;      // 0 idle, 1 refining, 2 accepted (at step cstep), 3 rejected, kPhaseFresh
     int cstep;      // step whose correction was accepted
     int xfinal;     // slot of the accepted X
     double max_e;   // largest correction of the last step
@@ -79,6 +79,10 @@ struct RefState {
     int live, pad;
 };
 constexpr int kMaxBackoff = 64;
+constexpr int kPhaseFresh = 4;  // slot V holds eigenvectors of this iteration's U (eig_big.hip)
+// Blocks up to kTriMaxRows have a tridiagonal eigensolver in one workgroup, the
+// larger ones, up to kBigMaxRows, that of eig_big.hip.
+constexpr int kTriMaxRows = 224, kBigMaxRows = 2048;
 
 struct RefDev {
     const RefBlock* blk;
@@ -87,7 +91,7 @@ struct RefDev {
     int* route;         // [global block]: how this iteration projects the block (kRoute*)
     double* work;
     double* part;
-    const double* tri_work;
+    double* tri_work;
     int nblk, njobs;
 };
 
@@ -125,6 +129,14 @@ void launch_ref_step(const BatchDev& B, const RefDev& R, const RefParams& P, int
 void launch_ref_final(const BatchDev& B, const RefDev& R, hipStream_t s);
 // Eigenvectors of the blocks that took the tridiagonal path this iteration.
 void launch_ref_form_v(const BatchDev& B, const RefDev& R, hipStream_t s);
+// x, z and sums of the blocks whose eigenvectors eig_big.hip just computed.
+void launch_ref_fresh(const BatchDev& B, const RefDev& R, hipStream_t s);
+// eig_big.hip: which of the n blocks list[] need the eigensolver, and the
+// eigenvectors of those (max_d: the largest of them); returns its launches.
+void launch_big_need(const BatchDev& B, const RefDev& R, const int* list, int n, bool refined, int* need,
+                     hipStream_t s);
+int launch_big_eig(const BatchDev& B, const RefDev& R, const int* list, const int* need, int n, int max_d,
+                   hipStream_t s);
 void launch_ref_forget(const RefDev& R, int blk_begin, int blk_end, hipStream_t s);
 
 // Blocks of up to 64 rows (refine_small.hip): one launch does the whole
@@ -159,6 +171,11 @@ class Refiner {
     void refine(const BatchDev& B, hipStream_t s) const;
     // kernel launches of begin() + refine(): state, sym, four per step, middle factor, final product and close
     int launches() const { return 5 + 4 * params_.max_steps; }
+    // Projection of the blocks above kTriMaxRows that the refinement has not
+    // taken (refined), or of all of them; the former waits for the refinement on
+    // the host.  Returns the kernel launches.
+    bool has_big() const { return !big_.empty(); }
+    int project_big(const BatchDev& B, bool refined, hipStream_t s);
     // After the fallback: eigenvectors of the blocks it projected.
     void seed(const BatchDev& B, hipStream_t s) const;
     void forget(int inst, hipStream_t s) const;
@@ -167,7 +184,7 @@ class Refiner {
     // divergence, for the correction size, for coupled clusters]
     static constexpr int kStats = 6;
     void stats(int64_t* out) const;
-    void set_work_base(const double* tri_work) { tri_work_ = tri_work; }
+    void set_work_base(double* tri_work) { tri_work_ = tri_work; }
     void set_params(const RefParams& p) { params_ = p; }
     const RefParams& params() const { return params_; }
 
@@ -182,7 +199,10 @@ class Refiner {
     DBuf<RefState> d_rs_;
     DBuf<int> route_;
     DBuf<double> work_, part_;
-    const double* tri_work_ = nullptr;
+    double* tri_work_ = nullptr;
+    std::vector<int> big_, need_host_;  // blocks above kTriMaxRows
+    int big_max_ = 0;
+    DBuf<int> d_big_, need_;
 };
 
 }  // namespace v2h

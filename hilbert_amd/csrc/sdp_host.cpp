@@ -80,6 +80,7 @@ void CallbackSdp::project(double* x) {
             proj_.launch(k, B, stream_);
         }
     }
+    if (proj_.has_big()) proj_.project_big(B, stream_);
     if (refine) proj_.refine_seed(B, stream_);
     V2H_HIP(hipGetLastError());
     V2H_HIP(hipMemcpyAsync(x, d_x_.p, bytes, hipMemcpyDeviceToHost, stream_));

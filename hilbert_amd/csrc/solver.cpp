@@ -863,7 +863,8 @@ int Batch::solve(int maxiter, const Monitor& mon) {
             // of tuning_.class_lane, joined back into stream_ (lock-step)
             launch_projection(Bx, seed, g);
         };
-        if (g < 0 && tuning_.graphs == kGraphAll) {
+        if (g < 0 && tuning_.graphs == kGraphAll && !proj_.has_big()) {
+            // (blocks above kTriMaxRows are looked at by the host: no capture)
             // the graph joins every lane it forks, so the eigenvector formation
             // (off the critical path) goes into the next CG graph
             run_graph(g_post_, graph_key(proj_.refine_on() ? "post_r" : "post"), [&] { post_projection(false); });
@@ -1004,6 +1005,13 @@ void Batch::launch_projection(const BatchDev& B, bool seed, int g) {
                 launches_++;
             }
         }
+    }
+    if (proj_.has_big()) {  // after the refinement, on its lane; the others are under way
+        if (!used[rl]) V2H_HIP(hipStreamWaitEvent(rs, E.post, 0));
+        used[rl] = true;
+        tstart(4 + kProjClasses - 1, rs);
+        launches_ += proj_.project_big(B, rs);
+        tstop(4 + kProjClasses - 1, rs);
     }
     if (g >= 0) {
         // the group's next pre waits for these events (wait_projection); the

@@ -178,15 +178,15 @@ class Batch {
     hipStream_t stream() const { return stream_; }
 
     // HIP-event timing of every kernel launch of solve(), per kernel kind:
-    // 0 pre, 1 cg_at, 2 cg_a, 3 post, 4..10 projection classes: Jacobi d <= 16,
-    // tridiagonal d <= 64 / 128 / 192 / 224 / 256, Jacobi d > 256 (matrix in
-    // global memory); 11: the device part of one set_df_integrals (its
+    // 0 pre, 1 cg_at, 2 cg_a, 3 post, 4..10 projection classes: d <= 16 (timed
+    // with the next where a batch has both), d <= 64 with its refinement, the
+    // tridiagonal eigensolver of d <= 128 / 192 / 224, (unused), d > 224; 11: the device part of one set_df_integrals (its
     // contraction kernels and the cost packing); 12: the pair Gram matrix of
     // write_fcidump; 13: the device work of optimize_orbitals outside the
     // intake (densities, Fock and Hessian products, exponential, transform);
-    // 14: the warm-started refinement of the 65..256 blocks (all its launches
+    // 14: the warm-started refinement of the blocks above 64 rows (all its launches
     // of one outer iteration); 15: the eigenvector formation of the blocks
-    // that fell back to the tridiagonal path.  Classes 2..5 then time only
+    // that fell back to the tridiagonal path.  Classes 2..4 then time only
     // their fallback launches.
     static constexpr int kProjClasses = Projector::kClasses;
     static constexpr int kKindDf = 4 + kProjClasses;
@@ -205,12 +205,12 @@ class Batch {
     // steps of a larger first chunk are skipped by the instances that have
     // stopped): what the autotuner (hilbert_amd/autotune.py) chooses.
     struct Tuning {
-        // lane (0 = stream_, 1..3 side streams) of each size class (Jacobi
-        // <= 16, tri 64 / 128 / 192 / 224 / 256, Jacobi > 256) when it is not
-        // refined, chosen to balance the per-iteration class times of the
+        // lane (0 = stream_, 1..3 side streams) of each size class (<= 16, 64,
+        // 128, 192, 224, 256 rows, > 256; the last two run on refine_lane)
+        // when it is not refined, chosen to balance the per-iteration class times of the
         // (16e,16o) workloads
         int class_lane[kProjClasses] = {0, 0, 2, 3, 1, 1, 2};
-        // lanes of the tridiagonal fallback of the refined classes (2..5)
+        // lanes of the tridiagonal fallback of the refined classes (2..4)
         int fallback_lane[kProjClasses] = {0, 0, 2, 3, 3, 2, 2};
         int refine_lane = 1;  // the warm-started refinement and the eigenvector formation (1..3)
         int cg_margin = 2;    // first CG chunk: the largest previous CG step count + cg_margin
@@ -227,8 +227,8 @@ class Batch {
     };
     void set_tuning(const Tuning& t);
     const Tuning& tuning() const { return tuning_; }
-    // Refined projection of the 65..256 blocks on (default) or off (every
-    // block takes the tridiagonal eigensolver).
+    // Refined projection on (default) or off (every block takes its
+    // eigensolver).
     void set_refine(bool on);
     bool refine() const { return proj_.refine_on(); }
     // [block projections by the refinement, by the fallback, rejections for

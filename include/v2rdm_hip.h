@@ -272,8 +272,8 @@ int v2h_batch_Au_noalloc(v2h_batch *b, int inst, const double *u, double *out);
 /* HIP-event timing of the kernels launched by v2h_batch_solve, recorded on
  * the library's stream.  ms[16] and counts[16] per kernel kind: 0 iteration
  * start (A [c - z, x, A^T y]), 1 CG A^T p, 2 CG A q, 3 A^T y and U, 4..10 PSD
- * projection classes: Jacobi for blocks up to 16, tridiagonal for blocks up to
- * 64 / 128 / 192 / 224 / 256, Jacobi beyond 256 (matrix in global memory);
+ * projection classes by rows: up to 16 (launched with the next), up to
+ * 64 / 128 / 192 / 224, up to 256 (launched with the next), above 224;
  * 11 the device part of v2h_batch_set_df_integrals (from the first
  * contraction kernel to the packed c), 12 the pair Gram matrix of
  * v2h_batch_write_fcidump, 13 the device work of v2h_batch_optimize_orbitals

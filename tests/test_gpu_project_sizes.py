@@ -62,6 +62,17 @@ SMALL = [1, 2, 3, 4, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64]
 @pytest.mark.parametrize("kind", ["plain", "degenerate", "zero", "positive", "negative"])
 @pytest.mark.parametrize("dims", [SMALL, [5, 16, 1], [20, 32, 7]], ids=["to64", "to16", "to32"])
 def test_projection_sequence(kind, dims):
+    _check(kind, dims)
+
+
+@pytest.mark.parametrize("kind", ["plain", "positive", "negative"])
+@pytest.mark.parametrize("dims", [[65, 96, 97, 128], [129, 192, 193, 224], [225, 256, 257], [2, 300, 64, 417]],
+                         ids=["to128", "to224", "to257", "mixed"])
+def test_projection_sequence_large(kind, dims):
+    _check(kind, dims)
+
+
+def _check(kind, dims):
     rng = np.random.default_rng([len(dims), len(kind)])
     seqs = [_sequence(kind, d, rng) for d in dims]
     n = sum(d * d for d in dims)
