@@ -68,7 +68,11 @@ CONV = [5e-8, 5e-7]
 
 
 def bytes_per_instance(kind, n_p, n_d):
-    """Algorithmic HBM bytes one launch moves for one instance."""
+    """HBM bytes of the vectors of one launch for one instance, as the plain
+    recurrences with w = A q stored have them (the count that earlier figures
+    and the traffic records use; the kernels now read r and q and write q in
+    cg_at, and read q and read and write r, p, y in cg_a: 8 (2 n_p + n_d) and
+    8 (n_p + 6 n_d))."""
     return 8 * {"cg_at": n_p + 3 * n_d,        # write q; read r, w, p
                 "cg_a": n_p + 8 * n_d,         # read q; read+write y, r, p, w
                 "pre": 3 * n_p + 5 * n_d,      # read c-z, x, A^T y; write 3; read b, y

@@ -61,7 +61,7 @@ struct InstState {
     double mu, bnorm, cnorm;
     double e_primal, e_dual, eps_p, eps_d;
     double cg_thr;              // tau^2 ||rhs||^2 of the current CG solve
-    double rr, pw, rw, ww;      // CG scalars of the last matvec
+    double rr, al, be;          // CG: |r|^2, step length and direction update of the current step
     int64_t oiter, iiter;
     int cg_iter, cg_done, cg_last;
     int active, converged, pending, status;  // pending: a projection awaits its bookkeeping
@@ -86,11 +86,10 @@ struct SolverOptions {
     double cg_tol_factor = kCgTolFactor;  // the factor of the CG stopping rule above
 };
 
-// CG state of one dual row, stored together so that a gather of the row
-// touches one 32-byte sector: residual r, w = A A^T p, direction p, dual y.
-struct alignas(32) CgRow {
-    double r, w, p, y;
-};
+// Counters by which the last workgroup of an instance knows that it is the
+// last: one per instance and one per kTicketGroup workgroups, each on a line of
+// its own (ints apart).
+constexpr int kTicketGroup = 32, kTicketStride = 32;
 
 // Batch-wide device arrays.
 struct BatchDev {
@@ -99,11 +98,12 @@ struct BatchDev {
     InstState* st;
     // primal-length arrays
     double *x, *z, *c, *v1, *u, *aty, *q;
-    // dual-length arrays
-    CgRow* cg;
-    double *av1, *ax, *aaty;
+    // dual-length arrays: residual and direction of the CG, dual y, and the two
+    // pieces of the first residual r = d0 + mu e (d0 = A (c - z) - A A^T y, e = b - A x)
+    double *r, *p, *y, *d0, *e;
     // reductions
     double* partials;       // per-workgroup partial dot products
+    int* ticket;            // counters of the instances, then of their groups of workgroups
     double* proj_part;      // per-block projection partials (c.x, dual residual)
     SolverOptions opt;
     // Instances a projection launch covers: every active one (pgroup < 0, the

@@ -1,11 +1,10 @@
 // kernels.hip -- CDNA4 (gfx950) kernels of the batched BPSDP solve.
 //
 // * Gather kernels over SELL-64 tables (one wavefront per 64 rows, or per
-//   long row).  Every CG step is three launches:
-//     k_cg_at     : q = A^T p, with p = (r - alpha w) + beta p formed on the fly
-//     k_cg_a      : w = A q, own-row updates of y, r, p, per-workgroup dot partials
-//     k_cg_reduce : one workgroup per instance sums the partials in a fixed
-//                   order (deterministic) and advances the CG state
+//   long row).  Every CG step is two launches, k_cg_at and k_cg_a, whose last
+//   workgroup of an instance sums the partial dot products in a fixed order
+//   (deterministic) and advances the CG state; k_cg_init forms the first
+//   residual.
 // * k_pre (+ k_pre_reduce): A [v1, x, A^T y] in one pass (rhs pieces, A x),
 //   then the end-of-iteration bookkeeping (errors, energies, mu, convergence,
 //   CG threshold).
@@ -54,27 +53,6 @@ __device__ __forceinline__ int unit_wg(const UnitsDev& U) {
             hi = mid;
     }
     return U.plan[U.plan_m + 1 + lo] + (c - U.plan[lo]);
-}
-
-// The CG vector recurrences, shared by the gather (on the fly) and the
-// owning-row update so both produce identical bits.
-__device__ __forceinline__ double r0_of(double av1, double b, double ax, double aaty, double mu) {
-    return __fma_rn(mu, b - ax, av1) - aaty;
-}
-__device__ __forceinline__ double r_next(double r, double w, double al) { return __fma_rn(-al, w, r); }
-__device__ __forceinline__ double p_next(double rn, double p, double be) { return __fma_rn(be, p, rn); }
-
-struct CgScalars {
-    double al, be;
-};
-__device__ __forceinline__ CgScalars cg_scalars(const InstState& st) {
-    CgScalars s{0.0, 0.0};
-    if (st.cg_iter > 0) {
-        s.al = st.rr / st.pw;
-        double rr1 = st.rr - 2.0 * s.al * st.rw + s.al * s.al * st.ww;
-        s.be = rr1 / st.rr;
-    }
-    return s;
 }
 
 // Gather over one SELL slice (lane = row) or one long row (whole wave).
@@ -235,7 +213,91 @@ __device__ __forceinline__ void put_coef(double* coef, double v) {
     __syncthreads();
 }
 
-// CG step, part 1: q = A^T p
+// Draws a ticket; true for the last of n, which takes the counter back to 0.
+__device__ __forceinline__ bool draw_last(int* t, int n) {
+    if (__hip_atomic_fetch_add(t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != n - 1) return false;
+    __hip_atomic_store(t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
+// Sum over the workgroups of one instance of v (each workgroup's over its
+// threads, in LDS red[4]) within the launch that produces it: the partial
+// value goes past the XCDs' L2s to memory, then the workgroup draws a ticket of
+// its group of 32, the last of a group one of the instance, and the very last
+// sums the nwg partial values in a fixed order.  True in that workgroup, whose
+// threads then all hold the total in v.  Every workgroup of the instance must
+// call it.  One launch less per reduction than a reducing kernel (4 to 5 us each
+// on an idle GPU, two per CG step).  Tickets of one counter are drawn one after
+// the other (about 12 ns each): with one per instance, 1900 workgroups took 25 us
+// longer, and 32 counters on one line 130 us for 24 000.
+__device__ __forceinline__ bool last_sum(const BatchDev& B, const UnitsDev& U, int inst, int wg, double* red,
+                                         double& v) {
+    __shared__ int last;
+    const int wg0 = U.wg_begin[inst], nwg = U.wg_begin[inst + 1] - wg0;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    v = wave_sum(v);
+    if (lane == 0) red[wv] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(B.partials + wg, (red[0] + red[1]) + (red[2] + red[3]), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the value has reached memory
+        const int grp = (wg - wg0) / kTicketGroup, ngrp = (nwg + kTicketGroup - 1) / kTicketGroup;
+        const int size = min(kTicketGroup, nwg - grp * kTicketGroup);
+        // groups of an instance from wg0 / kTicketGroup + inst on: no two share a counter
+        int* t = B.ticket + (size_t)(U.ninst + wg0 / kTicketGroup + inst + grp) * kTicketStride;
+        last = draw_last(t, size) && draw_last(B.ticket + (size_t)inst * kTicketStride, ngrp);
+    }
+    __syncthreads();
+    if (!last) return false;
+    double s = 0.0;
+    for (int k = threadIdx.x; k < nwg; k += kWG)
+        s += __hip_atomic_load(B.partials + wg0 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s = wave_sum(s);
+    if (lane == 0) red[wv] = s;
+    __syncthreads();
+    v = (red[0] + red[1]) + (red[2] + red[3]);
+    return true;
+}
+
+// The CG on A A^T y = A (c - z) + mu (b - A x), warm-started, with two launches
+// and two reductions per step:
+//   k_cg_at   q <- A^T r + beta q (= A^T p); alpha = |r|^2 / |q|^2
+//   k_cg_a    w = A q; p <- r + beta p, y <- y + alpha p, r <- r - alpha w;
+//             beta = |r|^2 / |r_old|^2, stop test
+// |q|^2 = p . A A^T p, so alpha is known before w: w is never stored, and the
+// gather of A^T reads 8 contiguous bytes per row (r) instead of r, w and p (24 of
+// a 32-byte row) to form p on the fly.  Per step and instance 8 (3 n_p + 7 n_d)
+// bytes of vectors instead of 8 (2 n_p + 12 n_d).  Bound by HBM (and L2 for the
+// gathers) in large batches, by launch latency for one small SDP.
+
+// r = d0 + mu e, |r|^2
+__global__ __launch_bounds__(kWG) void k_cg_init(BatchDev B, UnitsDev U) {
+    const int wg = unit_wg(U);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int inst = U.wg_inst[wg];
+    const UnitRec R = U.rec[(size_t)wg * 4 + wv];
+    InstState& st = B.st[inst];
+    if (!st.active || st.cg_done) return;
+    __shared__ double red[4];
+    // the slices cover every row (the long ones too, as lanes of theirs)
+    const bool in = (R.meta & kRecLong) == 0u && lane < (int)((R.meta >> 16) & 0x7Fu);
+    double rr = 0.0;
+    if (in) {
+        const int64_t g = B.inst[inst].doff + R.row + lane;
+        const double r = __fma_rn(st.mu, B.e[g], B.d0[g]);
+        B.r[g] = r;
+        rr = r * r;
+    }
+    if (!last_sum(B, U, inst, wg, red, rr) || threadIdx.x != 0) return;
+    st.rr = rr;
+    if (!isfinite(rr)) st.status |= kStatusNonFinite;
+    if (!(rr > st.cg_thr) || !isfinite(rr) || B.opt.cg_maxiter <= 0) {
+        st.cg_done = 1;
+        st.cg_last = 0;
+    }
+}
+
 __global__ __launch_bounds__(kWG) void k_cg_at(BatchDev B, UnitsDev U) {
     static_assert(kWG == 256, "one coefficient per thread");
     const int wg = unit_wg(U);
@@ -244,36 +306,42 @@ __global__ __launch_bounds__(kWG) void k_cg_at(BatchDev B, UnitsDev U) {
     const UnitRec R = U.rec[(size_t)wg * 4 + wv];
     const double cv = R.coef[threadIdx.x];
     WaveGather G(R, lane);
-    const InstState& st = B.st[inst];
+    InstState& st = B.st[inst];
     const InstDev I = B.inst[inst];
     if (!st.active || st.cg_done) return;
     __shared__ double coef[256];
+    __shared__ double red[4];
     put_coef(coef, cv);
-    const CgScalars cs = cg_scalars(st);
-    const double mu = st.mu;
+    const double be = st.be;
+    const bool first = st.cg_iter == 0;
+    double* q = B.q + I.poff;
+    const int64_t r0 = G.lane_row();
+    double qo = (!first && r0 >= 0) ? q[r0] : 0.0;  // loaded with the gather
+    const double* r = B.r + I.doff;
     double acc = 0.0;
-    int64_t row;
-    if (st.cg_iter == 0) {
-        const double *av1 = B.av1 + I.doff, *ax = B.ax + I.doff, *aaty = B.aaty + I.doff;
-        const double* b = B.structs[I.sid].b;
-        row = G.run(coef, [&](uint32_t col, double cf) {
-            acc = __fma_rn(cf, r0_of(av1[col], b[col], ax[col], aaty[col], mu), acc);
-        });
-    } else {
-        const CgRow* cg = B.cg + I.doff;
-        row = G.run(coef, [&](uint32_t col, double cf) {
-            const double2 rw = *reinterpret_cast<const double2*>(&cg[col].r);
-            acc = __fma_rn(cf, p_next(r_next(rw.x, rw.y, cs.al), cg[col].p, cs.be), acc);
-        });
-    }
+    int64_t row = G.run(coef, [&](uint32_t col, double cf) { acc = __fma_rn(cf, r[col], acc); });
     if (G.is_long) {
         acc = wave_sum(acc);
         if (lane != 0) row = -1;
+        if (!first && row >= 0) qo = q[row];
     }
-    if (row >= 0) B.q[I.poff + row] = acc;
+    double qq = 0.0;
+    if (row >= 0) {
+        const double qn = first ? acc : __fma_rn(be, qo, acc);
+        q[row] = qn;
+        qq = qn * qn;
+    }
+    if (!last_sum(B, U, inst, wg, red, qq) || threadIdx.x != 0) return;
+    if (!isfinite(qq)) st.status |= kStatusNonFinite;
+    if (qq > 0.0 && isfinite(qq)) {
+        st.al = st.rr / qq;
+    } else {  // r is in the null space of A^T: nothing left to reduce
+        st.cg_done = 1;
+        st.cg_last = st.cg_iter;
+        st.iiter += st.cg_iter;
+    }
 }
 
-// CG step, part 2: w = A q, own-row updates of y, r, p and the dot partials.
 __global__ __launch_bounds__(kWG) void k_cg_a(BatchDev B, UnitsDev U) {
     const int wg = unit_wg(U);
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -281,82 +349,64 @@ __global__ __launch_bounds__(kWG) void k_cg_a(BatchDev B, UnitsDev U) {
     const UnitRec R = U.rec[(size_t)wg * 4 + wv];
     const double cv = R.coef[threadIdx.x];
     WaveGather G(R, lane);
-    const InstState& st = B.st[inst];
+    InstState& st = B.st[inst];
     const InstDev I = B.inst[inst];
     if (!st.active || st.cg_done) return;
     __shared__ double coef[256];
-    __shared__ double red[4 * 4];
+    __shared__ double red[4];
     put_coef(coef, cv);
-    const CgScalars cs = cg_scalars(st);
-    const double mu = st.mu;
-    const int s = st.cg_iter;
+    const double al = st.al, be = st.be;
+    const bool first = st.cg_iter == 0;
     // the own row's state is loaded with the gather
     const int64_t r0 = G.lane_row();
-    CgRow c{0.0, 0.0, 0.0, 0.0};
-    if (r0 >= 0) c = B.cg[I.doff + r0];
+    double r = 0.0, p = 0.0, y = 0.0;
+    if (r0 >= 0) {
+        const int64_t g = I.doff + r0;
+        r = B.r[g];
+        y = B.y[g];
+        if (!first) p = B.p[g];
+    }
     const double* q = B.q + I.poff;
     double acc = 0.0;
     int64_t row = G.run(coef, [&](uint32_t col, double cf) { acc = __fma_rn(cf, q[col], acc); });
     if (G.is_long) {
         acc = wave_sum(acc);
         if (lane != 0) row = -1;
-        if (row >= 0) c = B.cg[I.doff + row];
+        if (row >= 0) {
+            const int64_t g = I.doff + row;
+            r = B.r[g];
+            y = B.y[g];
+            if (!first) p = B.p[g];
+        }
     }
-    double d4[4] = {0.0, 0.0, 0.0, 0.0};
+    double rr = 0.0;
     if (row >= 0) {
         const int64_t g = I.doff + row;
-        double rn, pn;
-        if (s == 0) {
-            rn = r0_of(B.av1[g], B.structs[I.sid].b[row], B.ax[g], B.aaty[g], mu);
-            pn = rn;
-        } else {
-            c.y = __fma_rn(cs.al, c.p, c.y);
-            rn = r_next(c.r, c.w, cs.al);
-            pn = p_next(rn, c.p, cs.be);
-        }
-        c.r = rn;
-        c.w = acc;
-        c.p = pn;
-        B.cg[g] = c;
-        d4[0] = rn * rn;
-        d4[1] = pn * acc;
-        d4[2] = rn * acc;
-        d4[3] = acc * acc;
+        const double pn = first ? r : __fma_rn(be, p, r);
+        const double rn = __fma_rn(-al, acc, r);
+        B.p[g] = pn;
+        B.y[g] = __fma_rn(al, pn, y);
+        B.r[g] = rn;
+        rr = rn * rn;
     }
-    block_partials<4>(d4, red, B.partials + (size_t)wg * 4);
-}
-
-// CG step, part 3 (one workgroup per instance): reduce the dots of k_cg_a and
-// advance the CG state.
-__global__ __launch_bounds__(kWG) void k_cg_reduce(BatchDev B, UnitsDev U) {
-    const int inst = blockIdx.x;
-    InstState& st = B.st[inst];
-    if (!st.active || st.cg_done || !in_pgroup(B, inst)) return;
-    __shared__ double red[4 * 4];
-    const int s = st.cg_iter;
-    double tot[4];
-    reduce_partials<4>(B.partials + (size_t)U.wg_begin[inst] * 4, U.wg_begin[inst + 1] - U.wg_begin[inst], red, tot);
-    if (threadIdx.x == 0) {
-        st.rr = tot[0];
-        st.pw = tot[1];
-        st.rw = tot[2];
-        st.ww = tot[3];
-        bool go_on = (s < B.opt.cg_maxiter) && (tot[0] > st.cg_thr) && (tot[1] > 0.0);
-        if (!isfinite(tot[0]) || !isfinite(tot[1])) {
-            st.status |= kStatusNonFinite;
-            go_on = false;
-        }
-        if (go_on) {
-            st.cg_iter = s + 1;
-        } else {
-            st.cg_done = 1;
-            st.cg_last = s;
-            st.iiter += s;
-        }
+    if (!last_sum(B, U, inst, wg, red, rr) || threadIdx.x != 0) return;
+    const int s = st.cg_iter + 1;
+    bool go_on = rr > st.cg_thr && s < B.opt.cg_maxiter;
+    if (!isfinite(rr)) {
+        st.status |= kStatusNonFinite;
+        go_on = false;
+    }
+    st.be = rr / st.rr;
+    st.rr = rr;
+    st.cg_iter = s;
+    if (!go_on) {
+        st.cg_done = 1;
+        st.cg_last = s;
+        st.iiter += s;
     }
 }
 
-// Start of an outer iteration: A [v1, x, aty] -> av1, ax, aaty; finishes the
+// Start of an outer iteration: A [v1, x, aty] -> d0, e; finishes the
 // previous iteration (errors, energies, mu, convergence) and sets up the CG.
 __global__ __launch_bounds__(kWG) void k_pre(BatchDev B, UnitsDev U) {
     const int wg = unit_wg(U);
@@ -387,15 +437,14 @@ __global__ __launch_bounds__(kWG) void k_pre(BatchDev B, UnitsDev U) {
     double d4[4] = {0.0, 0.0, 0.0, 0.0};
     if (row >= 0) {
         const int64_t g = I.doff + row;
-        B.av1[g] = a0;
-        B.ax[g] = a1;
-        B.aaty[g] = a2;
         const double bv = B.structs[I.sid].b[row];
         const double e = bv - a1;
+        B.d0[g] = a0 - a2;
+        B.e[g] = e;
         d4[0] = a0 * a0;
         d4[1] = a0 * e;
         d4[2] = e * e;
-        d4[3] = bv * B.cg[g].y;
+        d4[3] = bv * B.y[g];
     }
     block_partials<4>(d4, red, B.partials + (size_t)wg * 4);
 }
@@ -446,6 +495,7 @@ __global__ __launch_bounds__(kWG) void k_pre_reduce(BatchDev B, UnitsDev U) {
         double mu = st.mu;
         double rhs2 = tot[0] + 2.0 * mu * tot[1] + mu * mu * tot[2];
         st.cg_thr = tol * tol * rhs2;
+        st.be = 0.0;
         st.cg_iter = 0;
         st.cg_done = 0;
     }
@@ -464,9 +514,9 @@ __global__ __launch_bounds__(kWG) void k_post(BatchDev B, UnitsDev U) {
     if (!st.active) return;
     __shared__ double coef[256];
     put_coef(coef, cv);
-    const CgRow* cg = B.cg + I.doff;
+    const double* y = B.y + I.doff;
     double acc = 0.0;
-    int64_t row = G.run(coef, [&](uint32_t col, double cf) { acc = __fma_rn(cf, cg[col].y, acc); });
+    int64_t row = G.run(coef, [&](uint32_t col, double cf) { acc = __fma_rn(cf, y[col], acc); });
     if (G.is_long) {
         acc = wave_sum(acc);
         if (lane != 0) row = -1;
@@ -515,11 +565,6 @@ __global__ void k_fill(double* p, int64_t n, double v) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int64_t st = (int64_t)gridDim.x * blockDim.x;
     for (; i < n; i += st) p[i] = v;
-}
-
-__global__ void k_copy_strided(double* dst, int64_t dst_stride, const double* src, int64_t src_stride, int64_t n) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        dst[i * dst_stride] = src[i * src_stride];
 }
 
 __global__ void k_copy(double* dst, const double* src, int64_t n) {
@@ -583,10 +628,11 @@ __global__ __launch_bounds__(256) void k_dot_final(double* out) {
 void launch_cg_at(const BatchDev& B, const UnitsDev& U, hipStream_t s) {
     if (U.grid > 0) hipLaunchKernelGGL(k_cg_at, dim3(U.grid), dim3(kWG), 0, s, B, U);
 }
+void launch_cg_init(const BatchDev& B, const UnitsDev& U, hipStream_t s) {
+    if (U.grid > 0) hipLaunchKernelGGL(k_cg_init, dim3(U.grid), dim3(kWG), 0, s, B, U);
+}
 void launch_cg_a(const BatchDev& B, const UnitsDev& U, hipStream_t s) {
-    if (U.grid <= 0) return;
-    hipLaunchKernelGGL(k_cg_a, dim3(U.grid), dim3(kWG), 0, s, B, U);
-    hipLaunchKernelGGL(k_cg_reduce, dim3(U.ninst), dim3(kWG), 0, s, B, U);
+    if (U.grid > 0) hipLaunchKernelGGL(k_cg_a, dim3(U.grid), dim3(kWG), 0, s, B, U);
 }
 void launch_pre(const BatchDev& B, const UnitsDev& U, hipStream_t s) {
     // every instance: k_pre_reduce also finishes the bookkeeping of instances
@@ -610,11 +656,6 @@ static int grid_for(int64_t n) {
 
 void launch_fill(double* p, int64_t n, double v, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_fill, dim3(grid_for(n)), dim3(256), 0, s, p, n, v);
-}
-void launch_copy_strided(double* dst, int64_t dst_stride, const double* src, int64_t src_stride, int64_t n,
-                         hipStream_t s) {
-    if (n > 0)
-        hipLaunchKernelGGL(k_copy_strided, dim3(grid_for(n)), dim3(256), 0, s, dst, dst_stride, src, src_stride, n);
 }
 void launch_copy(double* dst, const double* src, int64_t n, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_copy, dim3(grid_for(n)), dim3(256), 0, s, dst, src, n);

@@ -149,16 +149,15 @@ Batch::Batch(const std::vector<ProblemDesc>& descs, const SolverOptions& opt, in
     build_projection();
 
     for (auto* b : {&x_, &z_, &c_, &v1_, &u_, &aty_, &q_}) b->alloc(np_total_);
-    for (auto* b : {&av1_, &ax_, &aaty_}) b->alloc(nd_total_);
-    cg_.alloc(nd_total_);
+    for (auto* b : {&r_, &p_, &y_, &d0_, &e_}) b->alloc(nd_total_);
+    ticket_.upload(std::vector<int>((2 * (size_t)N + std::max(nwgA_, nwgAT_) / kTicketGroup + 1) * kTicketStride, 0));
     src_.alloc(ns_total_);
     partials_.alloc(4 * (size_t)std::max(nwgA_, nwgAT_) + 4);
     int64_t smax = 0;
     for (const auto& s : structs_) smax = std::max({smax, s->n_primal, s->n_dual, s->nsrc});
     scratch_.alloc(std::max<int64_t>(2 * smax, 257));  // launch_dot1 needs 1 + 256
     for (auto* b : {&x_, &z_, &c_, &v1_, &u_, &aty_, &q_}) launch_fill(b->p, np_total_, 0.0, stream_);
-    for (auto* b : {&av1_, &ax_, &aaty_}) launch_fill(b->p, nd_total_, 0.0, stream_);
-    launch_fill(reinterpret_cast<double*>(cg_.p), 4 * nd_total_, 0.0, stream_);
+    for (auto* b : {&r_, &p_, &y_, &d0_, &e_}) launch_fill(b->p, nd_total_, 0.0, stream_);
     launch_fill(src_.p, ns_total_, 0.0, stream_);
 
     std::vector<StructDev> sd;
@@ -293,7 +292,8 @@ BatchDev Batch::dev() const {
     B.inst = d_inst_.p;
     B.st = d_state_.p;
     B.x = x_.p; B.z = z_.p; B.c = c_.p; B.v1 = v1_.p; B.u = u_.p; B.aty = aty_.p; B.q = q_.p;
-    B.cg = cg_.p; B.av1 = av1_.p; B.ax = ax_.p; B.aaty = aaty_.p;
+    B.r = r_.p; B.p = p_.p; B.y = y_.p; B.d0 = d0_.p; B.e = e_.p;
+    B.ticket = ticket_.p;
     B.partials = partials_.p;
     B.proj_part = proj_.proj_part();
     B.opt = opt_;
@@ -707,7 +707,7 @@ void Batch::set_guess_hf(int i) {
 void Batch::reset_state(int i) {
     const InstDev& I = inst_[i];
     const Structure& S = *structs_[inst_sid_[i]];
-    launch_fill(reinterpret_cast<double*>(cg_.p + I.doff), 4 * S.n_dual, 0.0, stream_);
+    launch_fill(y_.p + I.doff, S.n_dual, 0.0, stream_);
     launch_fill(z_.p + I.poff, S.n_primal, 0.0, stream_);
     launch_fill(aty_.p + I.poff, S.n_primal, 0.0, stream_);
     launch_copy(v1_.p + I.poff, c_.p + I.poff, S.n_primal, stream_);
@@ -764,7 +764,7 @@ int Batch::solve(int maxiter, const Monitor& mon) {
     for (int i = 0; i < count(); i++) seen[i] = state_[i].oiter;
 
     int cg_est[3] = {4, 4, 4};  // first CG chunk of group 0, group 1, the whole batch
-    for (const auto& st : state_) cg_est[2] = std::max(cg_est[2], st.cg_last + tuning_.cg_margin);
+    for (const auto& st : state_) cg_est[2] = std::max(cg_est[2], st.cg_last + tuning_.cg_margin - 1);
     cg_est[0] = cg_est[1] = cg_est[2];
     // timer attribution: a launch covers the whole batch only in lock-step
     auto refresh_flags = [&](int g) {
@@ -788,8 +788,9 @@ int Batch::solve(int maxiter, const Monitor& mon) {
         select(g, false);  // the instances running, as far as the host knows
         tstart(0);
         launch_pre(Bx, units_a(), stream_);
+        launch_cg_init(Bx, units_a(), stream_);
         tstop(0);
-        launches_++;
+        launches_ += 2;
         if (mon) {
             sync_state_to_host();
             for (int i = 0; i < count(); i++)
@@ -851,7 +852,7 @@ int Batch::solve(int maxiter, const Monitor& mon) {
         if (!any_active) return false;
         est = 4;
         for (int i = 0; i < count(); i++)
-            if (in_group(i, g)) est = std::max(est, state_[i].cg_last + tuning_.cg_margin);
+            if (in_group(i, g)) est = std::max(est, state_[i].cg_last + tuning_.cg_margin - 1);
         all_iterating_ = all_running_;  // the next CG solve starts for every running instance
         select(g, false);
         auto post_projection = [&](bool seed) {
@@ -1145,13 +1146,7 @@ static void h2d(double* dst, const double* src, int64_t n, hipStream_t s) {
 }
 
 void Batch::get_primal(int i, double* x) { d2h(x, x_.p + inst_[i].poff, n_primal(i), stream_); }
-// y is the fourth field of the CG rows: gathered into a contiguous buffer
-void Batch::get_dual(int i, double* y) {
-    DBuf<double> t;
-    t.alloc(n_dual(i));
-    launch_copy_strided(t.p, 1, &cg_.p[inst_[i].doff].y, 4, n_dual(i), stream_);
-    d2h(y, t.p, n_dual(i), stream_);
-}
+void Batch::get_dual(int i, double* y) { d2h(y, y_.p + inst_[i].doff, n_dual(i), stream_); }
 void Batch::get_slack(int i, double* z) { d2h(z, z_.p + inst_[i].poff, n_primal(i), stream_); }
 void Batch::get_cost(int i, double* c) { d2h(c, c_.p + inst_[i].poff, n_primal(i), stream_); }
 void Batch::get_b(int i, double* b) const {
@@ -1161,14 +1156,11 @@ void Batch::get_b(int i, double* b) const {
 void Batch::set_dual(int i, const double* y) {
     const Structure& S = *structs_[inst_sid_[i]];
     const InstDev& I = inst_[i];
-    DBuf<double> t;
-    t.alloc(n_dual(i));
-    h2d(t.p, y, n_dual(i), stream_);
-    launch_copy_strided(&cg_.p[I.doff].y, 4, t.p, 1, n_dual(i), stream_);
+    h2d(y_.p + I.doff, y, n_dual(i), stream_);
     // the next outer iteration starts from A (A^T y): keep aty = A^T y with y
     launch_fill(aty_.p + I.poff, S.n_primal, 0.0, stream_);
-    launch_spmv_plain(S.dev().AT, unitsAT_.p, hwgAT_begin_[i], hwgAT_begin_[i + 1] - hwgAT_begin_[i], t.p,
-                      aty_.p + I.poff, stream_);
+    launch_spmv_plain(S.dev().AT, unitsAT_.p, hwgAT_begin_[i], hwgAT_begin_[i + 1] - hwgAT_begin_[i],
+                      y_.p + I.doff, aty_.p + I.poff, stream_);
     V2H_HIP(hipStreamSynchronize(stream_));
 }
 void Batch::set_slack(int i, const double* z) {

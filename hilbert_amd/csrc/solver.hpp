@@ -305,8 +305,8 @@ class Batch {
     DBuf<StructDev> d_structs_;
     DBuf<InstDev> d_inst_;
     DBuf<InstState> d_state_;
-    DBuf<double> x_, z_, c_, v1_, u_, aty_, q_, av1_, ax_, aaty_;
-    DBuf<CgRow> cg_;
+    DBuf<double> x_, z_, c_, v1_, u_, aty_, q_, r_, p_, y_, d0_, e_;
+    DBuf<int> ticket_;
     DBuf<double> src_, partials_, scratch_;
     DBuf<int4> unitsA_, unitsAT_;        // work-unit codes (per-instance maps)
     DBuf<UnitRec> recA_, recAT_;          // the same units, resolved (batched gathers)
