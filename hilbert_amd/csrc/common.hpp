@@ -38,8 +38,19 @@ struct SellDev {
     int nslices, nlong;
 };
 
+// Pieces of one operator (sell.hpp); only for structures whose CG runs in one
+// workgroup.
+struct PieceDev {
+    const uint32_t* ent;
+    const uint32_t* slice;
+    const int32_t* dst;
+    const int32_t* multi;
+    int nslices, nmulti;
+};
+
 struct StructDev {
     SellDev A, AT;
+    PieceDev pA, pAT;
     const double* b;        // [n_dual]
     const int32_t* cost1;   // [n_primal] cost-vector gather map
     const int32_t* cost2;
@@ -53,7 +64,12 @@ struct InstDev {
     int64_t soff;           // offset into the batch integral array [h; g]
     int sid;                // structure id
     int block_first, nblocks;
+    int small;              // its CG runs in one workgroup (k_cg_small)
 };
+
+// An instance is small when r, q and the partial sums of its CG fit in the LDS
+// of one workgroup beside two coefficient tables (160 KB).
+constexpr int64_t kSmallCgDoubles = 20480 - 2 * 256 - 32;
 
 // Per-instance solver state, written only by the reducing workgroup of a
 // kernel (the last one to finish) or by the host between launches.

@@ -11,11 +11,14 @@
 // * k_post : A^T y and U = mu x + A^T y - c.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "sell.hpp"
+#include "wave_ops.hpp"
 
 namespace v2h {
 
@@ -278,7 +281,7 @@ __global__ __launch_bounds__(kWG) void k_cg_init(BatchDev B, UnitsDev U) {
     const int inst = U.wg_inst[wg];
     const UnitRec R = U.rec[(size_t)wg * 4 + wv];
     InstState& st = B.st[inst];
-    if (!st.active || st.cg_done) return;
+    if (!st.active || st.cg_done || B.inst[inst].small) return;
     __shared__ double red[4];
     // the slices cover every row (the long ones too, as lanes of theirs)
     const bool in = (R.meta & kRecLong) == 0u && lane < (int)((R.meta >> 16) & 0x7Fu);
@@ -308,7 +311,7 @@ __global__ __launch_bounds__(kWG) void k_cg_at(BatchDev B, UnitsDev U) {
     WaveGather G(R, lane);
     InstState& st = B.st[inst];
     const InstDev I = B.inst[inst];
-    if (!st.active || st.cg_done) return;
+    if (!st.active || I.small || st.cg_done) return;
     __shared__ double coef[256];
     __shared__ double red[4];
     put_coef(coef, cv);
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(kWG) void k_cg_a(BatchDev B, UnitsDev U) {
     WaveGather G(R, lane);
     InstState& st = B.st[inst];
     const InstDev I = B.inst[inst];
-    if (!st.active || st.cg_done) return;
+    if (!st.active || I.small || st.cg_done) return;
     __shared__ double coef[256];
     __shared__ double red[4];
     put_coef(coef, cv);
@@ -403,6 +406,168 @@ __global__ __launch_bounds__(kWG) void k_cg_a(BatchDev B, UnitsDev U) {
         st.cg_done = 1;
         st.cg_last = s;
         st.iiter += s;
+    }
+}
+
+// A slice of pieces (sell.hpp) in the registers of a wavefront.
+struct PieceSlice {
+    uint32_t e[kPiece];
+    int32_t dst;
+    int w;
+    __device__ __forceinline__ void load(const PieceDev& T, int u, int lane) {
+        w = 0;
+        dst = kNoPiece;
+#pragma unroll
+        for (int k = 0; k < kPiece; k++) e[k] = 0u;
+        if (u >= T.nslices) return;
+        const uint32_t s = T.slice[u];
+        w = (int)(s >> 28);
+        dst = T.dst[u * 64 + lane];
+        const uint32_t* p = T.ent + (s & 0x0FFFFFFFu) + lane;
+#pragma unroll
+        for (int k = 0; k < kPiece; k++)
+            if (k < w) e[k] = p[64 * k];
+    }
+    // (the empty asm keeps the addresses, which no step changes, from being held
+    // in registers too)
+    __device__ __forceinline__ double sum(const double* coef, const double* v) const {
+        uint32_t x[kPiece];
+#pragma unroll
+        for (int k = 0; k < kPiece; k++) {
+            x[k] = e[k];
+            asm volatile("" : "+v"(x[k]));
+        }
+        double a = coef[x[0] >> 24] * v[x[0] & 0xFFFFFFu];
+        if (w > 1) {  // (uniform)
+            const double b = coef[x[1] >> 24] * v[x[1] & 0xFFFFFFu];
+            if (w > 2) {
+                a = __fma_rn(coef[x[2] >> 24], v[x[2] & 0xFFFFFFu], a);
+                a = __fma_rn(coef[x[3] >> 24], v[x[3] & 0xFFFFFFu], a);
+            }
+            a += b;
+        }
+        return a;
+    }
+};
+
+// The whole CG of a small instance (list[blockIdx.x]) in one workgroup, r, q and
+// partial sums in LDS: a step is two passes over the pieces of the gather
+// tables, each with a pass over the rows of several pieces and a workgroup sum;
+// no step is launched that is not needed and the host looks at no CG.  A
+// wavefront has at most kSmallHeld slices in each direction and keeps them and
+// its rows' p and y in registers, so nothing but LDS is read in a step: beyond
+// that (streaming the slices from L2) a step takes as long as its two launches
+// would.  Bound by the latency of the LDS gathers, barriers and sums: (6e,6o) C2v,
+// 22 steps, 118 us, against 310 us in two launches a step and 222 us streaming.
+constexpr int kSmallNT = 1024, kSmallHeld = 6;
+__global__ __launch_bounds__(kSmallNT) void k_cg_small(BatchDev B, const int* list) {
+    extern __shared__ double sm[];
+    constexpr int NW = kSmallNT / 64, KU = kSmallHeld;
+    const int inst = list[blockIdx.x];
+    InstState& st = B.st[inst];
+    if (!st.active || !in_pgroup(B, inst)) return;
+    const InstDev I = B.inst[inst];
+    const StructDev& S = B.structs[I.sid];
+    const PieceDev TA = S.pA, TT = S.pAT;
+    const int nd = (int)S.n_dual;
+    double *coefA = sm, *coefT = sm + 256, *red = sm + 512, *r = sm + 544, *q = r + nd, *part = q + S.n_primal;
+    double* Y = B.y + I.doff;
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    int half = 0;  // alternating sum buffers: one barrier per sum
+    auto wg_sum = [&](double v) {
+        double* b = red + 16 * half;
+        half ^= 1;
+        v = wsum(v);
+        if (lane == 0) b[wv] = v;
+        __syncthreads();
+        double s4[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < NW; k++) s4[k & 3] += b[k];
+        return (s4[0] + s4[1]) + (s4[2] + s4[3]);
+    };
+    if (t < 256) {
+        coefA[t] = S.A.coef[t];
+        coefT[t] = S.AT.coef[t];
+    }
+    PieceSlice hA[KU], hT[KU];
+    double yh[KU], ph[KU], ym = 0.0, pm = 0.0;  // of the held pieces' rows and of multi row t
+#pragma unroll
+    for (int m = 0; m < KU; m++) {
+        hA[m].load(TA, wv + NW * m, lane);
+        hT[m].load(TT, wv + NW * m, lane);
+        yh[m] = hA[m].dst >= 0 ? Y[hA[m].dst] : 0.0;
+        ph[m] = 0.0;
+    }
+    // the multi rows of the two operators that are this thread's
+    int3 mA = make_int3(-1, 0, 0), mT = mA;
+    if (t < TA.nmulti) mA = make_int3(TA.multi[3 * t], TA.multi[3 * t + 1], TA.multi[3 * t + 2]);
+    if (t < TT.nmulti) mT = make_int3(TT.multi[3 * t], TT.multi[3 * t + 1], TT.multi[3 * t + 2]);
+    if (mA.x >= 0) ym = Y[mA.x];
+    const double mu = st.mu, thr = st.cg_thr;
+    double rr = 0.0;
+    for (int i = t; i < nd; i += kSmallNT) {
+        const double v = __fma_rn(mu, B.e[I.doff + i], B.d0[I.doff + i]);
+        r[i] = v;
+        rr = __fma_rn(v, v, rr);
+    }
+    rr = wg_sum(rr);
+    // one(row, sum, p, y) for every row of the operator applied to v
+    auto apply = [&](const PieceSlice(&h)[KU], const int3& mr, bool multi, const double* coef, const double* v,
+                     auto&& one) {
+#pragma unroll
+        for (int m = 0; m < KU; m++) {
+            if (h[m].w == 0) continue;  // (uniform)
+            const double a = h[m].sum(coef, v);
+            int dst = h[m].dst;
+            asm volatile("" : "+v"(dst));
+            if (dst >= 0) one(dst, a, ph[m], yh[m]);
+            else if (dst != kNoPiece) part[-1 - dst] = a;
+        }
+        if (!multi) return;
+        __syncthreads();
+        if (mr.x >= 0) {
+            double a = part[mr.y];
+            for (int k = 1; k < mr.z; k++) a += part[mr.y + k];
+            one(mr.x, a, pm, ym);
+        }
+    };
+    double be = 0.0;
+    int s = 0, bad = !isfinite(rr);
+    while (!bad && rr > thr && s < B.opt.cg_maxiter) {
+        double qq = 0.0;
+        apply(hT, mT, TT.nmulti > 0, coefT, r, [&](int row, double a, double&, double&) {
+            const double qn = s > 0 ? __fma_rn(be, q[row], a) : a;
+            q[row] = qn;
+            qq = __fma_rn(qn, qn, qq);
+        });
+        qq = wg_sum(qq);
+        bad = !isfinite(qq);
+        if (bad || !(qq > 0.0)) break;  // 0: r is in the null space of A^T
+        const double al = rr / qq;
+        double rn2 = 0.0;
+        apply(hA, mA, TA.nmulti > 0, coefA, q, [&](int row, double a, double& p, double& y) {
+            const double ro = r[row], rn = __fma_rn(-al, a, ro);
+            p = s > 0 ? __fma_rn(be, p, ro) : ro;
+            y = __fma_rn(al, p, y);
+            r[row] = rn;
+            rn2 = __fma_rn(rn, rn, rn2);
+        });
+        rn2 = wg_sum(rn2);
+        be = rn2 / rr;
+        rr = rn2;
+        s++;
+        bad = !isfinite(rr);
+    }
+#pragma unroll
+    for (int m = 0; m < KU; m++)
+        if (hA[m].dst >= 0) Y[hA[m].dst] = yh[m];
+    if (mA.x >= 0) Y[mA.x] = ym;
+    if (t == 0) {
+        if (bad) st.status |= kStatusNonFinite;
+        st.rr = rr;
+        st.cg_iter = st.cg_last = s;
+        st.iiter += s;
+        st.cg_done = 1;
     }
 }
 
@@ -630,6 +795,17 @@ void launch_cg_at(const BatchDev& B, const UnitsDev& U, hipStream_t s) {
 }
 void launch_cg_init(const BatchDev& B, const UnitsDev& U, hipStream_t s) {
     if (U.grid > 0) hipLaunchKernelGGL(k_cg_init, dim3(U.grid), dim3(kWG), 0, s, B, U);
+}
+bool cg_small_fits(int a_slices, int at_slices, int a_multi, int at_multi) {
+    return std::max(a_slices, at_slices) <= kSmallHeld * (kSmallNT / 64) && std::max(a_multi, at_multi) <= kSmallNT;
+}
+void launch_cg_small(const BatchDev& B, const int* list, int n, int64_t vec_doubles, hipStream_t s) {
+    const size_t lds = sizeof(double) * (size_t)(vec_doubles + 544);
+    static_assert(kSmallCgDoubles + 544 <= 160 * 1024 / 8, "one workgroup's LDS");
+    if (n > 0) hipLaunchKernelGGL(k_cg_small, dim3(n), dim3(kSmallNT), lds, s, B, list);
+}
+void set_cg_small_lds_limit() {
+    V2H_HIP(hipFuncSetAttribute((const void*)k_cg_small, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
 }
 void launch_cg_a(const BatchDev& B, const UnitsDev& U, hipStream_t s) {
     if (U.grid > 0) hipLaunchKernelGGL(k_cg_a, dim3(U.grid), dim3(kWG), 0, s, B, U);

@@ -10,6 +10,12 @@
 namespace v2h {
 
 void launch_cg_init(const BatchDev& B, const UnitsDev& U, hipStream_t s);  // U: the units of A
+// The CG of the n small instances list[] (those running); vec_doubles: the most
+// LDS doubles that one of them needs (n_primal + n_dual + the partial sums of the
+// wider operator).  cg_small_fits: whether an operator's pieces fit the registers.
+bool cg_small_fits(int a_slices, int at_slices, int a_multi, int at_multi);
+void launch_cg_small(const BatchDev& B, const int* list, int n, int64_t vec_doubles, hipStream_t s);
+void set_cg_small_lds_limit();
 void launch_cg_at(const BatchDev& B, const UnitsDev& U, hipStream_t s);
 void launch_cg_a(const BatchDev& B, const UnitsDev& U, hipStream_t s);
 void launch_pre(const BatchDev& B, const UnitsDev& U, hipStream_t s);

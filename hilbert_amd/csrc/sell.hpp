@@ -32,4 +32,22 @@ struct SellHost {
 
 SellHost build_sell(const Csr& M, int long_threshold);
 
+// The same operator cut into pieces of at most kPiece entries of one row, for
+// the workgroup that keeps a whole small operator to itself: wide rows would
+// leave it waiting for one wavefront.  64 pieces of like length make a slice
+// (entries k-major, coefficient codes of S); dst of a piece is its row, or for
+// a row of several pieces -1 - position of its partial sum.
+constexpr int kPiece = 4;
+struct PieceHost {
+    std::vector<uint32_t> ent;
+    std::vector<uint32_t> slice;   // first entry | width << 28
+    std::vector<int32_t> dst;      // [slices][64], kNoPiece where there is none
+    std::vector<int32_t> multi;    // rows of several pieces: row, first position, pieces (3 each)
+    int nparts = 0;
+    int nslices() const { return (int)slice.size(); }
+    int nmulti() const { return (int)multi.size() / 3; }
+};
+constexpr int32_t kNoPiece = INT32_MIN;
+PieceHost build_pieces(const Csr& M, const SellHost& S);
+
 }  // namespace v2h

@@ -49,6 +49,15 @@ Structure::Structure(const ProblemDesc& d) : L(d) {
     hAT = build_sell(AT, kLongThreshold);
     unitsA = unit_list(hA);
     unitsAT = unit_list(hAT);
+    if (n_primal + n_dual <= kSmallCgDoubles) {
+        const PieceHost pa = build_pieces(A, hA), pt = build_pieces(AT, hAT);
+        const int64_t need = n_primal + n_dual + std::max(pa.nparts, pt.nparts);
+        if (need <= kSmallCgDoubles && cg_small_fits(pa.nslices(), pt.nslices(), pa.nmulti(), pt.nmulti())) {
+            small_doubles = need;
+            a_pieces.upload(pa);
+            at_pieces.upload(pt);
+        }
+    }
 
     CostMap cm = build_cost_map(L);
     const int64_t n = L.n;
@@ -77,8 +86,19 @@ Structure::Structure(const ProblemDesc& d) : L(d) {
     adj_ent.upload(ent);
 }
 
+void Structure::Pieces::upload(const PieceHost& h) {
+    ent.upload(h.ent);
+    slice.upload(h.slice);
+    dst.upload(h.dst);
+    multi.upload(h.multi);
+    nslices = h.nslices();
+    nmulti = h.nmulti();
+}
+
 StructDev Structure::dev() const {
     StructDev s{};
+    s.pA = a_pieces.dev();
+    s.pAT = at_pieces.dev();
     s.A = SellDev{a_ent.p, a_slice.p, a_lstart.p, a_lent.p, a_lrow.p, a_coef.p, hA.nrows, hA.nslices, hA.nlong()};
     s.AT = SellDev{at_ent.p, at_slice.p, at_lstart.p, at_lent.p, at_lrow.p, at_coef.p, hAT.nrows, hAT.nslices,
                    hAT.nlong()};
@@ -108,6 +128,8 @@ Batch::Batch(const std::vector<ProblemDesc>& descs, const SolverOptions& opt, in
     }
     V2H_HIP(hipEventCreateWithFlags(&ev_seed_, hipEventDisableTiming));
     V2H_HIP(hipEventCreateWithFlags(&ev_gfork_, hipEventDisableTiming));
+    V2H_HIP(hipEventCreateWithFlags(&ev_sfork_, hipEventDisableTiming));
+    V2H_HIP(hipEventCreateWithFlags(&ev_sjoin_, hipEventDisableTiming));
     V2H_HIP(hipEventCreateWithFlags(&ev_joined_, hipEventDisableTiming));
     V2H_HIP(hipEventCreateWithFlags(&ev_gjoin_, hipEventDisableTiming));
     for (auto& row : ev_pdone_)
@@ -141,10 +163,17 @@ Batch::Batch(const std::vector<ProblemDesc>& descs, const SolverOptions& opt, in
         inst_[i].doff = nd_total_;
         inst_[i].soff = ns_total_;
         inst_[i].sid = inst_sid_[i];
+        if (S.small_doubles > 0) {
+            inst_[i].small = 1;
+            small_.push_back(i);
+            small_doubles_ = std::max(small_doubles_, S.small_doubles);
+        }
         np_total_ += S.n_primal;
         nd_total_ += S.n_dual;
         ns_total_ += S.nsrc;
     }
+    d_small_.upload(small_);
+    if (!small_.empty()) set_cg_small_lds_limit();
     build_units();
     build_projection();
 
@@ -210,7 +239,8 @@ Batch::~Batch() {
             if (e) (void)hipEventDestroy(e);
     }
     if (ev_seed_) (void)hipEventDestroy(ev_seed_);
-    if (ev_gfork_) (void)hipEventDestroy(ev_gfork_);
+    for (hipEvent_t e : {ev_gfork_, ev_sfork_, ev_sjoin_})
+        if (e) (void)hipEventDestroy(e);
     if (ev_joined_) (void)hipEventDestroy(ev_joined_);
     if (ev_gjoin_) (void)hipEventDestroy(ev_gjoin_);
     for (auto& row : ev_pdone_)
@@ -764,7 +794,8 @@ int Batch::solve(int maxiter, const Monitor& mon) {
     for (int i = 0; i < count(); i++) seen[i] = state_[i].oiter;
 
     int cg_est[3] = {4, 4, 4};  // first CG chunk of group 0, group 1, the whole batch
-    for (const auto& st : state_) cg_est[2] = std::max(cg_est[2], st.cg_last + tuning_.cg_margin - 1);
+    for (int i = 0; i < count(); i++)
+        if (!inst_[i].small) cg_est[2] = std::max(cg_est[2], state_[i].cg_last + tuning_.cg_margin - 1);
     cg_est[0] = cg_est[1] = cg_est[2];
     // timer attribution: a launch covers the whole batch only in lock-step
     auto refresh_flags = [&](int g) {
@@ -777,6 +808,8 @@ int Batch::solve(int maxiter, const Monitor& mon) {
     refresh_flags(-1);
     all_iterating_ = all_running_;
 
+    constexpr int kUnseen = 8;  // outer iterations of small instances between two looks at their state
+    int unseen = 0;
     // One outer iteration of group g (g < 0: the whole batch) on stream_:
     // pre, the CG in chunks with host polls, post and the projection.
     // Returns false when none of its instances runs any more.
@@ -786,11 +819,13 @@ int Batch::solve(int maxiter, const Monitor& mon) {
         refresh_flags(g);
         all_iterating_ = all_running_;
         select(g, false);  // the instances running, as far as the host knows
+        bool small = false, large = false;
+        for (int i = 0; i < count(); i++) (inst_[i].small ? small : large) |= in_group(i, g);
         tstart(0);
         launch_pre(Bx, units_a(), stream_);
-        launch_cg_init(Bx, units_a(), stream_);
+        if (large) launch_cg_init(Bx, units_a(), stream_);
         tstop(0);
-        launches_ += 2;
+        launches_ += large ? 2 : 1;
         if (mon) {
             sync_state_to_host();
             for (int i = 0; i < count(); i++)
@@ -799,10 +834,36 @@ int Batch::solve(int maxiter, const Monitor& mon) {
                     mon(i, status(i));
                 }
         }
+        if (small) {  // their whole CG, beside the others'
+            hipStream_t ss = large ? pstream_[kSideStreams - 1] : stream_;
+            if (large) {
+                V2H_HIP(hipEventRecord(ev_sfork_, stream_));
+                V2H_HIP(hipStreamWaitEvent(ss, ev_sfork_, 0));
+            }
+            tstart(1, ss);
+            launch_cg_small(Bx, d_small_.p, (int)small_.size(), small_doubles_, ss);
+            launches_++;
+            tstop(1, ss);
+            if (large) V2H_HIP(hipEventRecord(ev_sjoin_, ss));
+        }
         int steps = 0, chunk = est;
         bool any_active = true;
+        if (!large) {
+            // nothing for the host to decide: launches of an instance that has
+            // stopped do nothing, so it looks only now and then whether any runs
+            if (seed_owed_) {
+                launch_seed(Bx);
+                seed_owed_ = false;
+            }
+            if (mon || ++unseen >= kUnseen) {
+                unseen = 0;
+                sync_state_to_host();
+                refresh_flags(g);
+                any_active = running(g) > 0;
+            }
+        }
         const bool graphs = g < 0 && tuning_.graphs >= kGraphCg;
-        for (;;) {
+        while (large) {
             const UnitsDev UA = units_a(), UAT = units_at();
             // the eigenvector formation owed by a projection graph runs as a
             // branch beside the first chunk, joined at its end
@@ -843,16 +904,17 @@ int Batch::solve(int maxiter, const Monitor& mon) {
             any_active = false;
             for (int i = 0; i < count(); i++) {
                 any_active |= in_group(i, g);
-                pending |= in_group(i, g) && !state_[i].cg_done;
+                pending |= in_group(i, g) && !inst_[i].small && !state_[i].cg_done;
             }
             if (!pending || steps > opt_.cg_maxiter) break;
             select(g, true);  // the instances whose CG goes on
             chunk = 4;
         }
+        if (small && large) V2H_HIP(hipStreamWaitEvent(stream_, ev_sjoin_, 0));
         if (!any_active) return false;
         est = 4;
         for (int i = 0; i < count(); i++)
-            if (in_group(i, g)) est = std::max(est, state_[i].cg_last + tuning_.cg_margin - 1);
+            if (in_group(i, g) && !inst_[i].small) est = std::max(est, state_[i].cg_last + tuning_.cg_margin - 1);
         all_iterating_ = all_running_;  // the next CG solve starts for every running instance
         select(g, false);
         auto post_projection = [&](bool seed) {

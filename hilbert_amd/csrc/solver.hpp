@@ -33,6 +33,16 @@ struct Structure {
     DBuf<uint32_t> a_ent, a_slice, a_lstart, a_lent, at_ent, at_slice, at_lstart, at_lent;
     DBuf<int32_t> a_lrow, at_lrow, cost1, cost2, adj_ptr, adj_ent;
     DBuf<double> a_coef, at_coef, b_dev;
+    // the CG in one workgroup (k_cg_small): LDS doubles it needs, 0 where the
+    // structure is too large for it
+    int64_t small_doubles = 0;
+    struct Pieces {
+        DBuf<uint32_t> ent, slice;
+        DBuf<int32_t> dst, multi;
+        int nslices = 0, nmulti = 0;
+        void upload(const PieceHost& h);
+        PieceDev dev() const { return PieceDev{ent.p, slice.p, dst.p, multi.p, nslices, nmulti}; }
+    } a_pieces, at_pieces;
     StructDev dev() const;
 };
 
@@ -332,6 +342,13 @@ class Batch {
     bool pdone_used_[2][kSideStreams] = {};
     hipEvent_t ev_seed_ = nullptr;
     bool seed_pending_ = false;
+    // instances whose CG runs in one workgroup each (InstDev::small), the most
+    // LDS doubles that one of them needs, and the fork and join of their launch
+    // where it runs beside the others' CG
+    std::vector<int> small_;
+    DBuf<int> d_small_;
+    int64_t small_doubles_ = 0;
+    hipEvent_t ev_sfork_ = nullptr, ev_sjoin_ = nullptr;
 
     struct KTimer {
         std::vector<std::pair<hipEvent_t, hipEvent_t>> pool;  // every event pair of this kind
