@@ -21,10 +21,21 @@ void launch_dgemm(bool ta, bool tb, int M, int N, int K, double alpha, const dou
 // products in work, [slices][M][N], then summed in slice order): for a small
 // M x N with a long K.
 constexpr int kMaxSlices = 64;
-// C = alpha op(A) B (+ dg on the diagonal), beta = 0, one product; the LDS
-// kernel when M, N, K <= 128, else launch_dgemm.
+// C = alpha op(A) B (+ dg on the diagonal), beta = 0, one product; the
+// one-tile kernel when M, N, K <= 128, else launch_dgemm.
 void launch_dgemm_small(bool ta, int M, int N, int K, double alpha, const double* A, int64_t lda, const double* B,
                         int64_t ldb, double* C, int64_t ldc, hipStream_t s, double dg = 0.0);
+// Epilogue of the one-tile kernel: C = alpha op(A) B + c[0] I + c[1] M1 + c[2] M2 + c[3] M3,
+// and where Q is given also Q = q[0] I + q[1] M1 + q[2] M2 + q[3] C; a null matrix
+// counts as zero, all of C's shape and leading dimension.
+struct SmallPoly {
+    double c[4], q[4];
+    const double *M1, *M2, *M3;
+    double* Q;
+};
+// exp(K) of an n x n K with ||K||_1 <= 1/2; W: 3 n^2 doubles.  The result is in
+// U or in T, whichever is returned.
+double* launch_oo_exp_taylor(int n, const double* K, double* W, double* U, double* T, hipStream_t s);
 int dgemm_split_slices(int M, int N, int K);
 void launch_dgemm_split(bool ta, bool tb, int M, int N, int K, double alpha, const double* A, int64_t lda,
                         const double* B, int64_t ldb, double beta, double* C, int64_t ldc, double* work,
@@ -48,8 +59,9 @@ struct OoTables {
 void launch_oo_density(const OoTables& t, const double* x, double* D, double* d, hipStream_t s);
 
 // BO[Q][r][s] = B[Q][occ r][occ s], BFO[p][r][Q] = B[Q][p][occ r], Bdiag[p][Q] = B[Q][p][p]
-void launch_oo_gather(const double* bd, int nq, int nfull, const int* occ, int no, double* BO, double* BFO,
-                      double* Bdiag, hipStream_t s);
+// (pos: position of an orbital in occ, or -1)
+void launch_oo_gather(const double* bd, int nq, int nfull, const int* occ, int no, const int* pos, double* BO,
+                      double* BFO, double* Bdiag, hipStream_t s);
 
 // F[x][y] += sum_r D[x][r] h[y][occ r]
 void launch_oo_fock1(const double* D, const double* h, const int* occ, int no, int nfull, double* F,

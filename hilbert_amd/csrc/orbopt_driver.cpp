@@ -107,6 +107,7 @@ void Batch::oo_setup(int i, const OrbOptArgs& a) {
         S.bd.alloc((size_t)nq * nn);
         S.tmp.alloc((size_t)nq * nn);
         for (auto* b : {&S.uscr, &S.hscr, &S.K, &S.U, &S.T1}) b->alloc(nn);
+        S.W.alloc(3 * nn);
         S.D.alloc(n2);
         S.d.alloc(n2 * n2);
         S.gO.alloc(n2 * n2);
@@ -131,7 +132,7 @@ void Batch::oo_gradient(int i) {
     DfState& S = df_state(i);
     const int nfull = S.nfull, no = S.no, nq = S.nq, n2 = S.no * S.no;
     tstart(kKindOrb);
-    launch_oo_gather(S.bd.p, nq, nfull, S.occ.p, no, S.BO.p, S.BFO.p, S.Bdiag.p, stream_);
+    launch_oo_gather(S.bd.p, nq, nfull, S.occ.p, no, S.pos.p, S.BO.p, S.BFO.p, S.Bdiag.p, stream_);
     launch_dgemm_split(true, false, n2, n2, nq, 1.0, S.BO.p, n2, S.BO.p, n2, 0.0, S.gO.p, n2, S.Gw.p, stream_);
     launch_dgemm_split(false, true, n2, nq, n2, 1.0, S.d.p, n2, S.BO.p, n2, 0.0, S.Z.p, nq, S.Zw.p, stream_);
     launch_dgemm_split(false, true, no, nfull, no * nq, 1.0, S.Z.p, (int64_t)no * nq, S.BFO.p, (int64_t)no * nq, 0.0,
@@ -177,17 +178,9 @@ double Batch::oo_apply(int i, const double* kappa, double sign) {
     while (sq < 60 && nrm / std::ldexp(1.0, sq) > 0.5) sq++;
     tstart(kKindOrb);
     if (sq > 0) launch_oo_axpy(std::ldexp(1.0, -sq) - 1.0, S.K.p, S.K.p, nn, stream_);
-    // exp(K) on the scaled K: the Taylor polynomial of degree 14 by Horner's
-    // rule, T <- I + K T / k for k = 14 .. 1 (the identity added in the
-    // product's epilogue), then squared back
-    double* U = S.U.p;
-    double* T1 = S.T1.p;
-    launch_oo_identity(U, nfull, stream_);
-    constexpr int kTaylor = 14;
-    for (int k = kTaylor; k >= 1; k--) {
-        launch_dgemm_small(false, nfull, nfull, nfull, 1.0 / k, S.K.p, nfull, U, nfull, T1, nfull, stream_, 1.0);
-        std::swap(U, T1);
-    }
+    // the exponential of the scaled K, then squared back
+    double* U = launch_oo_exp_taylor(nfull, S.K.p, S.W.p, S.U.p, S.T1.p, stream_);
+    double* T1 = U == S.U.p ? S.T1.p : S.U.p;
     for (int k = 0; k < sq; k++) {
         launch_dgemm_small(false, nfull, nfull, nfull, 1.0, U, nfull, U, nfull, T1, nfull, stream_);
         std::swap(U, T1);
