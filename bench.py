@@ -79,7 +79,7 @@ def bytes_per_instance(kind, n_p, n_d):
                 "post": 4 * n_p + n_d}[kind]   # read y, x, c; write A^T y, U
 
 
-# with the refinement on, the 65..256 classes time only their fallback
+# with the refinement on, the classes above 64 rows time only their fallback
 # launches, so their work per launch is an upper bound
 PROJ_CLASSES = (("project_jacobi16", 0, 16), ("project_tri64", 17, 64), ("project_tri128", 65, 128),
                 ("project_tri192", 129, 192), ("project_tri224", 193, 224), ("project_tri256", 225, 256),
@@ -639,7 +639,7 @@ def main():
     ap.add_argument("--refine-steps", type=int, default=5,
                     help="refinement steps before a block falls back to the tridiagonal eigensolver")
     ap.add_argument("--projection", choices=("refined", "tridiagonal"), default="refined",
-                    help="PSD blocks of 65..256 rows: warm-started refinement on the FP64 matrix cores with the "
+                    help="PSD blocks: warm-started refinement on the FP64 matrix cores with the "
                          "tridiagonal fallback, or the tridiagonal eigensolver alone")
     args = ap.parse_args()
     PROGRESS_CHUNK[0] = max(1, args.chunk)

@@ -32,8 +32,8 @@ import time
 
 import numpy as np
 
-# (class_lane, fallback_lane, refine_lane) presets; classes: Jacobi <= 16,
-# tridiagonal <= 64 / 128 / 192 / 224 / 256, Jacobi > 256
+# (class_lane, fallback_lane, refine_lane) presets; classes by
+# rows: <= 16, 64, 128, 192, 224, 256, > 256
 LANE_PRESETS = {
     "balanced": ([0, 0, 2, 3, 1, 1, 2], [0, 0, 2, 3, 3, 2, 2], 1),
     "small_on_main": ([0, 0, 1, 2, 3, 3, 1], [0, 0, 2, 3, 2, 3, 3], 1),

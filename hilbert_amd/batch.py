@@ -299,10 +299,10 @@ class Batch:
     PROJECT_TRIDIAGONAL, PROJECT_REFINED = 0, 1
 
     def set_projection(self, mode):
-        """PROJECT_REFINED (default): blocks of 65..256 rows refine the
-        previous iteration's eigenvectors on the FP64 matrix cores and fall
-        back to the tridiagonal eigensolver; PROJECT_TRIDIAGONAL: always the
-        tridiagonal eigensolver."""
+        """PROJECT_REFINED (default): every block refines the previous
+        iteration's eigenvectors on the FP64 matrix cores and falls back to
+        the eigensolver of its size; PROJECT_TRIDIAGONAL: always the
+        eigensolver."""
         N.check(N.lib().v2h_batch_set_projection(self._h, int(mode)))
         self._projection = int(mode)
 

@@ -405,7 +405,7 @@ __global__ __launch_bounds__(256) void k_oo_fock1(const double* __restrict__ D, 
 }
 
 // One workgroup per rotation pair: its threads split the O^2 sums, combined in
-// a fixed order (1900 pairs with 26^2 terms: 9.5 us; 24 with a
+// a fixed order (573 pairs with 26^2 terms: 9.5 us; 24 with a
 // wavefront per pair).
 __global__ __launch_bounds__(256) void k_oo_grad_hess(OoGradArgs a) {
     __shared__ double part[4][4];

@@ -1010,8 +1010,9 @@ int Batch::solve(int maxiter, const Monitor& mon) {
 //
 // Without the refinement every size class starts right after k_post on its
 // lane (tuning_.class_lane) and stream_ joins the lanes.  With it, the lane
-// tuning_.refine_lane runs the warm-started refinement of the 65..256
-// classes: its first kernel sets each block's route, after which the
+// tuning_.refine_lane runs the warm-started refinement of the blocks above 64
+// rows (the smaller ones are refined by one launch on their own lane): its
+// first kernel sets each block's route, after which the
 // tridiagonal launches of the blocks known to need the fallback start on
 // their lanes (tuning_.fallback_lane) beside the refinement; after the
 // refinement the same lanes take the blocks it rejected.  stream_ joins every

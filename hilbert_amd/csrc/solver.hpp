@@ -250,7 +250,7 @@ class Batch {
     }
     void set_profiling(bool on) { profile_ = on; }
     // hipGraph replay of the fixed launch sequences of an outer iteration:
-    // kGraphCg, the first CG chunk (its k_cg_at / k_cg_a / k_cg_reduce
+    // kGraphCg, the first CG chunk (its k_cg_at / k_cg_a
     // launches); kGraphAll, also k_post with the whole projection (every size
     // class on its lane, the refinement and its fallback passes, joined into
     // stream_), the eigenvector formation then running as a branch of the

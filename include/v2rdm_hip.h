@@ -278,23 +278,25 @@ int v2h_batch_Au_noalloc(v2h_batch *b, int inst, const double *u, double *out);
  * contraction kernel to the packed c), 12 the pair Gram matrix of
  * v2h_batch_write_fcidump, 13 the device work of v2h_batch_optimize_orbitals
  * besides the intake (densities, Fock and Hessian products, exponential,
- * integral transform), 14 the warm-started refinement of the blocks of
- * 65..256 rows (all its launches of one outer iteration), 15 the eigenvector
- * formation of the blocks that took the tridiagonal fallback (with the
- * refinement on, kinds 6..9 time only the fallback launches).  Cumulative
+ * integral transform), 14 the warm-started refinement of the blocks above
+ * 64 rows (all its launches of one outer iteration), 15 the eigenvector
+ * formation of the blocks of 65..224 rows that took the tridiagonal fallback
+ * (with the refinement on, kinds 5..8 and 10 time the fallback launches, kind 5
+ * also the refinement of the blocks of up to 64 rows).  Cumulative
  * since the last reset.  full_ms / full_counts (may be NULL) cover only the launches
  * made while every instance was running (for CG kernels: still iterating)
  * at the previous host poll, i.e. launches that processed the whole batch. */
 int v2h_batch_set_profiling(v2h_batch *b, int on);
 /* hipGraph replay inside v2h_batch_solve (the graphs field of v2h_tuning):
  * mode 1 captures the first CG chunk of every outer iteration (its k_cg_at /
- * k_cg_a / k_cg_reduce launches) once per set of running instances and step
+ * k_cg_a launches) once per set of running instances and step
  * count and replays it with one hipGraphLaunch (with the kernel timers on,
  * v2h_batch_set_profiling, the launches go one by one); the results are the
  * bits of mode 0 (default, every kernel launched one by one).  Mode 2 also
  * captures k_post and the whole projection (forked onto the side streams and
  * joined back), with the eigenvector formation as a branch of the next CG
- * graph; the same bits again.
+ * graph; the same bits again.  A batch with a block above 224 rows, whose
+ * projection the host takes part in, keeps mode 1's graphs only.
  * The libsdp loop it replaces launches nothing (v2rdm_solver.cc:1305-1361). */
 int v2h_batch_set_graphs(v2h_batch *b, int mode);
 
@@ -306,11 +308,12 @@ int v2h_batch_set_graphs(v2h_batch *b, int mode);
  * reference, whose libsdp loop runs on the host. */
 typedef struct {
     int class_lane[7];    /* stream of each PSD size class when not refined:
-                           * Jacobi <= 16, tridiagonal <= 64 / 128 / 192 /
-                           * 224 / 256, Jacobi > 256; 0 = the batch's main
+                           * <= 16, 64, 128, 192, 224, 256, > 256 rows (the
+                           * first launched with the second, the last two on
+                           * the refinement's stream); 0 = the batch's main
                            * stream, 1..3 its side streams */
     int fallback_lane[7]; /* stream of the tridiagonal fallback of the refined
-                           * classes (entries 2..5 used) */
+                           * classes (entries 2..4 used) */
     int refine_lane;      /* side stream (1..3) of the refinement and the
                            * eigenvector formation */
     int cg_margin;        /* first CG chunk of an outer iteration: the largest
@@ -337,22 +340,21 @@ int v2h_batch_reset_kernel_times(v2h_batch *b);
  * A^T gather workgroups, projection blocks] */
 int v2h_batch_launch_stats(v2h_batch *b, int64_t *stats);
 
-/* How the PSD blocks of 65..256 rows are projected (the eigendecomposition
+/* How the PSD blocks are projected (the eigendecomposition
  * libsdp applies to every block of dimensions_, v2rdm_solver.cc:1340, block
  * list v2rdm_solver.cc:3729-3846):
  *   V2H_PROJECT_REFINED (default): the eigenvectors of the previous outer
  *     iteration are refined by FP64 matrix-core products (iterative
- *     refinement of Ogita and Aishima, at most five steps by default,
- *     accepted when the last correction is below 2e-7); blocks without
- *     eigenvectors yet, or
- *     whose refinement is not accepted, take the tridiagonal eigensolver,
- *     whose eigenvectors seed the next iteration;
- *   V2H_PROJECT_TRIDIAGONAL: every block takes the tridiagonal eigensolver.
- * Smaller and larger blocks are not affected. */
+ *     refinement of Ogita and Aishima, at most seven steps by default,
+ *     accepted when the last correction is below 2e-7, up to 64 rows 3e-8);
+ *     blocks without eigenvectors yet, or whose refinement is not accepted,
+ *     take the eigensolver (tridiagonal, up to 16 rows Jacobi), whose
+ *     eigenvectors seed the next iteration;
+ *   V2H_PROJECT_TRIDIAGONAL: every block takes the eigensolver. */
 #define V2H_PROJECT_TRIDIAGONAL 0
 #define V2H_PROJECT_REFINED 1
 int v2h_batch_set_projection(v2h_batch *b, int mode);
-/* Over the blocks of 65..256 rows since the batch was created: [block
+/* Over the blocks above 64 rows since the batch was created: [block
  * projections done by the refinement, by the tridiagonal fallback, refinements
  * rejected for a diverging or non-finite correction, for a correction still
  * above accept_e after max_steps steps, for clusters left coupled, FP64 flops
