@@ -223,6 +223,7 @@ __device__ __forceinline__ double tri_eigenvalue(int l, int d, const double* dd,
     }
     lam = 0.5 * (lo + hi);
     double last = INFINITY;
+    bool probed = false;
     while (passes < kMaxPasses) {
         if (hi - lo <= abstol) {
             lam = 0.5 * (lo + hi);
@@ -233,16 +234,36 @@ __device__ __forceinline__ double tri_eigenvalue(int l, int d, const double* dd,
         if (clo == l && chi == l + 1 && haveS) {
             const double step = -1.0 / S;
             sn = s + step;
+            const bool inside = sn > lo && sn < hi;
             if (fabs(step) <= 2.0 * abstol) {
-                lam = fmin(fmax(sn, lo), hi);
-                break;
+                if (inside) {
+                    lam = sn;
+                    break;
+                }
+                // Out of the bracket, by rounding at eigenvalue l or at a
+                // neighbour of it: next to one of high multiplicity S is large and
+                // the step small, however far eigenvalue l is.  A count across
+                // s tells (bisecting instead: 33 passes per eigenvalue of a random
+                // 224-row T, against 16).
+                if (!probed) {
+                    probed = true;
+                    const double x = s <= lo ? lo + 2.0 * abstol : hi - 2.0 * abstol;
+                    double Sx;
+                    if (x > lo && x < hi) eval(x, Sx);
+                    if (hi - lo <= 2.5 * abstol) {
+                        lam = 0.5 * (lo + hi);
+                        break;
+                    }
+                    continue;
+                }
             }
-            newton = isfinite(sn) && sn > lo && sn < hi && fabs(step) <= 0.5 * last;
+            newton = inside && fabs(step) <= 0.5 * last;
             if (newton) last = fabs(step);
         }
         if (!newton) {
             sn = 0.5 * (lo + hi);
             last = INFINITY;
+            probed = false;
         }
         s = sn;
         eval(s, S);

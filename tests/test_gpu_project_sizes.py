@@ -72,9 +72,49 @@ def test_projection_sequence_large(kind, dims):
     _check(kind, dims)
 
 
+def _degenerate_sequence(kind, d, rng):
+    """Blocks whose eigenvalues are equal in large groups, diagonal and turned,
+    some of them after a zero block (whose eigenvalues are the guess then)."""
+    def spectrum():
+        if kind == "ends":          # one eigenvalue at each end, two groups between
+            w = np.zeros(d)
+            w[1:1 + d // 2] = 1.0
+            w[0] = 2.0
+            w[-1] = -2.0 if d > 2 else w[-1]
+        elif kind == "integers":    # the cost of a caller's map, say
+            w = rng.integers(-2, 2, d).astype(float)
+            w[0] = 2.0
+        elif kind == "one":         # one positive, many zero, many negative
+            w = -rng.uniform(0.1, 1.0, d)
+            w[: (d + 1) // 2] = 0.0
+            w[0] = 1.0
+        else:                       # low rank
+            w = np.zeros(d)
+            w[: max(1, d // 20)] = rng.uniform(0.5, 1.0, max(1, d // 20))
+        return rng.permutation(w)
+
+    def turned(w):
+        Q = np.linalg.qr(rng.standard_normal((d, d)))[0]
+        U = (Q * w) @ Q.T
+        return 0.5 * (U + U.T)
+
+    return [np.diag(spectrum()), np.zeros((d, d)), turned(spectrum()), np.zeros((d, d)), np.diag(spectrum()),
+            turned(spectrum())]
+
+
+@pytest.mark.parametrize("kind", ["ends", "integers", "one", "rank"])
+@pytest.mark.parametrize("dims", [[17, 31, 32, 33, 47, 48, 49, 63, 64], [65, 96, 128, 224]], ids=["to64", "to224"])
+def test_projection_of_degenerate_blocks(kind, dims):
+    rng = np.random.default_rng([len(dims), len(kind), 1])
+    _check_sequences(kind, dims, [_degenerate_sequence(kind, d, rng) for d in dims])
+
+
 def _check(kind, dims):
     rng = np.random.default_rng([len(dims), len(kind)])
-    seqs = [_sequence(kind, d, rng) for d in dims]
+    _check_sequences(kind, dims, [_sequence(kind, d, rng) for d in dims])
+
+
+def _check_sequences(kind, dims, seqs):
     n = sum(d * d for d in dims)
     S = BPSDPSolver(n, 1, options(e_convergence=1e-30, r_convergence=1e-30, maxiter=10 ** 6))
     zero_a = lambda u: np.zeros(1)
