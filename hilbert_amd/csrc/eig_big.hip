@@ -12,7 +12,9 @@
 //                 to its own rows and multiplies them by the new v.  Row k is
 //                 read by all and rewritten by none, so a step needs no barrier
 //                 but its launch.
-//   T = S L S^T   one thread per eigenvalue, 64 per workgroup (tri_eigen.hpp)
+//   T = S L S^T   one thread per eigenvalue, 64 per workgroup (tri_eigen.hpp);
+//                 the vectors of a cluster of close eigenvalues are
+//                 orthogonalised by a workgroup
 //   V = Q S       compact-WY products of 16 reflectors, 64 columns per workgroup
 //   U+            the final product of the refinement, V being the accepted X
 //
@@ -218,23 +220,35 @@ __global__ __launch_bounds__(64) void k_big_values(BatchDev B, RefDev R, const i
     if (bad) atomicOr(&B.st[b.inst].status, (int)kStatusJacobiNotConverged);
 }
 
-// Eigenvectors of T, one thread per cluster of close eigenvalues.
-__global__ __launch_bounds__(64) void k_big_vectors(BatchDev B, RefDev R, const int* list, const int* need) {
+// ||T||, the same value in every lane (as k_big_values and the kernels below
+// need it: Gershgorin's bound on the largest |eigenvalue|).
+__device__ __forceinline__ double big_norm(const Area& W, int d) {
+    double m = 0.0;
+    for (int i = threadIdx.x & 63; i < d; i += 64)
+        m = fmax(m, fabs(W.dd[i]) + (i > 0 ? fabs(W.ee[i - 1]) : 0.0) + (i + 1 < d ? fabs(W.ee[i]) : 0.0));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    return m;
+}
+
+// Inverse iteration, one thread per eigenvector: the first solve or (second) the
+// one after it.  Between and after them k_big_ortho orthogonalises each
+// cluster: as in tri_vectors, except that a whole cluster takes each step
+// together.
+__global__ __launch_bounds__(64) void k_big_vectors(BatchDev B, RefDev R, const int* list, const int* need,
+                                                    int second) {
     __shared__ double dd[kMaxD], ee[kMaxD], lam[kMaxD];
     if (!need[blockIdx.y]) return;
     const RefBlock b = R.blk[list[blockIdx.y]];
     const int d = b.d, t = threadIdx.x, l = blockIdx.x * 64 + t;
     if ((int)blockIdx.x * 64 >= d) return;
     const Area W(R.tri_work, b);
-    double tnorm = 0.0;
+    const double tnorm = big_norm(W, d);
     for (int i = t; i < d; i += 64) {
         dd[i] = W.dd[i];
         ee[i] = i + 1 < d ? W.ee[i] : 0.0;
         lam[i] = W.lam[i];
-        tnorm = fmax(tnorm, fabs(W.dd[i]) + (i > 0 ? fabs(W.ee[i - 1]) : 0.0) + (i + 1 < d ? fabs(W.ee[i]) : 0.0));
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) tnorm = fmax(tnorm, __shfl_xor(tnorm, o, 64));
     __syncthreads();
     if (l >= d) return;
     if (!(tnorm > 0.0)) {  // T = 0: any orthonormal basis
@@ -242,12 +256,117 @@ __global__ __launch_bounds__(64) void k_big_vectors(BatchDev B, RefDev R, const 
         W.xs[l] = 1.0;
         return;
     }
-    if (tri_linked(lam, l, tnorm)) return;
-    int l1 = l;
-    while (l1 + 1 < d && tri_linked(lam, l1 + 1, tnorm)) l1++;
-    bool bad = false;
-    tri_vectors(l, l1, d, dd, ee, lam, W.xs, tnorm, W.S, W.fac, bad);
-    if (bad) atomicOr(&B.st[b.inst].status, (int)kStatusJacobiNotConverged);
+    const Column col{W.S + l, W.fac + l, (size_t)d, (size_t)d * d};
+    if (second) {
+        const double s2 = tri_resolve(col, d, W.xs[l]);
+        const bool bad = !(s2 > 0.0) || !isfinite(s2);
+        W.xs[l] = bad ? INFINITY : s2;
+        if (bad) atomicOr(&B.st[b.inst].status, (int)kStatusJacobiNotConverged);
+        return;
+    }
+    int l0 = l;
+    while (tri_linked(lam, l0, tnorm)) l0--;
+    double sg = -INFINITY;
+    for (int i = l0; i <= l; i++) sg = tri_shift(lam[i], sg, tnorm);
+    W.xs[l] = tri_solve(col, l, d, dd, ee, sg, tnorm);
+}
+
+// Gram-Schmidt, twice, of the vectors of every cluster of close eigenvalues;
+// workgroup g takes the clusters that begin at an eigenvalue 16 g .. 16 g + 15.
+// 16 columns at a time are orthogonalised against the earlier ones, 64 by 64
+// (coefficients of a wavefront per quarter of the rows, summed in LDS), then
+// among each other.  A cluster of m vectors takes about 8 m^2 d products and
+// reads its columns m / 16 times.  A whole projection of 300 rows: 3.8 ms, with
+// 200 equal eigenvalues 12.5 ms, with 285 of them 29 ms; of 417 rows with 397
+// equal ones 82 ms.  One thread per cluster, with dependent loads of single
+// values, takes 1.8 s for 213 equal ones of 224 rows.
+__global__ __launch_bounds__(kNT) void k_big_ortho(BatchDev B, RefDev R, const int* list, const int* need) {
+    constexpr int kP = 16, kE = 64;  // columns of a panel, earlier columns at a time
+    __shared__ double lam[kMaxD];
+    __shared__ double part[4][kP][kE], cf[kP][kE + 1], red[4];
+    if (!need[blockIdx.y]) return;
+    const RefBlock b = R.blk[list[blockIdx.y]];
+    const int d = b.d, t = threadIdx.x, lane = t & 63, w = t >> 6, q = t & 15, r = t >> 4;
+    if ((int)blockIdx.x * 16 >= d) return;
+    const Area W(R.tri_work, b);
+    double* S = W.S;
+    const double tnorm = big_norm(W, d);
+    if (!(tnorm > 0.0)) return;
+    for (int i = t; i < d; i += kNT) lam[i] = W.lam[i];
+    __syncthreads();
+    // (every branch and loop bound below is the same for the whole workgroup,
+    // but for the rows and columns of a thread)
+    for (int l0 = blockIdx.x * 16; l0 < min((int)blockIdx.x * 16 + 16, d); l0++) {
+        if (tri_linked(lam, l0, tnorm)) continue;
+        int l1 = l0;
+        while (l1 + 1 < d && tri_linked(lam, l1 + 1, tnorm)) l1++;
+        if (l1 == l0) continue;
+        for (int p0 = l0; p0 <= l1; p0 += kP) {
+            const int pb = min(kP, l1 + 1 - p0);
+            for (int pass = 0; pass < 2; pass++) {
+                for (int c0 = l0; c0 < p0; c0 += kE) {
+                    const int nc = min(kE, p0 - c0);
+                    double acc[kP];
+#pragma unroll
+                    for (int k = 0; k < kP; k++) acc[k] = 0.0;
+                    for (int i = w; i < d; i += 4) {
+                        const double* row = S + (size_t)i * d;
+                        const double y = lane < nc ? row[c0 + lane] : 0.0;
+#pragma unroll
+                        for (int k = 0; k < kP; k++) acc[k] = fma(y, row[min(p0 + k, d - 1)], acc[k]);
+                    }
+#pragma unroll
+                    for (int k = 0; k < kP; k++) part[w][k][lane] = acc[k];
+                    __syncthreads();
+                    for (int e = t; e < kP * kE; e += kNT) {
+                        const int k = e / kE, c = e % kE;
+                        const double s = (part[0][k][c] + part[1][k][c]) + (part[2][k][c] + part[3][k][c]);
+                        cf[k][c] = c < nc ? s / W.xs[c0 + c] : 0.0;
+                    }
+                    __syncthreads();
+                    if (q < pb)
+                        for (int i = r; i < d; i += kNT / 16) {
+                            double* row = S + (size_t)i * d;
+                            double v = row[p0 + q];
+                            for (int c = 0; c < nc; c++) v = fma(-cf[q][c], row[c0 + c], v);
+                            row[p0 + q] = v;
+                        }
+                    __syncthreads();
+                }
+                for (int k = 0; k < pb; k++) {  // column k of the panel against those before it
+                    if (k > 0) {
+                        double s = 0.0;
+                        if (q < k)
+                            for (int i = r; i < d; i += kNT / 16)
+                                s = fma(S[(size_t)i * d + p0 + q], S[(size_t)i * d + p0 + k], s);
+                        part[0][q][r] = s;
+                        __syncthreads();
+                        if (t < k) {
+                            s = 0.0;
+                            for (int e = 0; e < kNT / 16; e++) s += part[0][t][e];
+                            cf[0][t] = s / W.xs[p0 + t];
+                        }
+                        __syncthreads();
+                    }
+                    double s2 = 0.0;
+                    for (int i = t; i < d; i += kNT) {
+                        double* row = S + (size_t)i * d + p0;
+                        double v = row[k];
+                        for (int c = 0; c < k; c++) v = fma(-cf[0][c], row[c], v);
+                        row[k] = v;
+                        s2 = fma(v, v, s2);
+                    }
+                    s2 = wg_sum(s2, red);
+                    if (t == 0) {
+                        const bool bad = !(s2 > 0.0) || !isfinite(s2);
+                        W.xs[p0 + k] = bad ? INFINITY : s2;  // INFINITY drops the vector
+                        if (bad) atomicOr(&B.st[b.inst].status, (int)kStatusJacobiNotConverged);
+                    }
+                    __syncthreads();
+                }
+            }
+        }
+    }
 }
 
 // Triangular factor of H_kc .. H_kc+15 = I - Y T Y^T (dlarft forward order), one
@@ -384,10 +503,13 @@ int launch_big_eig(const BatchDev& B, const RefDev& R, const int* list, const in
     for (int k = 0; k <= max_d - 2; k++)
         hipLaunchKernelGGL(k_big_step, dim3(wgs, n), dim3(kNT), 0, s, R, list, need, k);
     hipLaunchKernelGGL(k_big_values, dim3(cols, n), dim3(64), 0, s, B, R, list, need);
-    hipLaunchKernelGGL(k_big_vectors, dim3(cols, n), dim3(64), 0, s, B, R, list, need);
+    for (int second = 0; second < 2; second++) {
+        hipLaunchKernelGGL(k_big_vectors, dim3(cols, n), dim3(64), 0, s, B, R, list, need, second);
+        hipLaunchKernelGGL(k_big_ortho, dim3((max_d + 15) / 16, n), dim3(kNT), 0, s, B, R, list, need);
+    }
     hipLaunchKernelGGL(k_big_wy, dim3(wy, n), dim3(kNT), 0, s, R, list, need);
     hipLaunchKernelGGL(k_big_form_v, dim3(cols, n), dim3(kNT), 0, s, R, list, need);
-    return max_d + 4;
+    return max_d + 7;
 }
 
 }  // namespace v2h

@@ -279,69 +279,85 @@ __device__ __forceinline__ bool tri_linked(const double* lamv, int l, double tno
     return l > 0 && (lamv[l] - lamv[l - 1]) <= kClusterRel * fmax(fabs(lamv[l]), fabs(lamv[l - 1])) + kClusterAbs * tnorm;
 }
 
+// Shift of the inverse iteration for eigenvector l: its eigenvalue, kept apart
+// from the shift before it in the cluster (sprev; -INFINITY at its first).
+__device__ __forceinline__ double tri_shift(double lam, double sprev, double tnorm) {
+    const double pert = 10.0 * kEps * fmax(fabs(lam), 1e-3 * tnorm);
+    return lam <= sprev + pert ? sprev + pert : lam;
+}
+
+// First solve for eigenvector l: T - sg I = P L U with partial pivoting
+// ([q][i]: 0 multiplier, 1 reciprocal pivot, 2-3 superdiagonals of U, 4
+// interchange), fused with L^{-1} P applied to the start vector; then U^{-1}.
+// Returns ||x||^2.
+__device__ __forceinline__ double tri_solve(const Column& col, int l, int d, const double* dd, const double* ee,
+                                            double sg, double tnorm) {
+    const double ptol = kEps * tnorm;
+    double dcur = dd[0] - sg, ucur = d > 1 ? ee[0] : 0.0;
+    double bc = start_value((uint32_t)l, 0u);
+    for (int i = 0; i + 1 < d; i++) {
+        const double sub = ee[i];
+        double dnext = dd[i + 1] - sg;
+        double unext = (i + 2 < d) ? ee[i + 1] : 0.0;
+        const double bn = start_value((uint32_t)l, (uint32_t)(i + 1));
+        double f, u0, u1, u2, sw, xi;
+        if (fabs(dcur) >= fabs(sub)) {
+            if (fabs(dcur) < ptol) dcur = (dcur < 0.0) ? -ptol : ptol;
+            f = sub * recip(dcur);
+            u0 = dcur;
+            u1 = ucur;
+            u2 = 0.0;
+            sw = 0.0;
+            dnext = fma(-f, ucur, dnext);
+            xi = bc;
+            bc = fma(-f, bc, bn);
+        } else {
+            f = dcur * recip(sub);
+            u0 = sub;
+            u1 = dnext;
+            u2 = unext;
+            sw = 1.0;
+            dnext = fma(-f, dnext, ucur);
+            unext = -f * unext;
+            xi = bn;
+            bc = fma(-f, bn, bc);
+        }
+        col.f(0, i) = f;
+        col.f(1, i) = recip(u0);
+        col.f(2, i) = u1;
+        col.f(3, i) = u2;
+        col.f(4, i) = sw;
+        col.X(i) = xi;
+        dcur = dnext;
+        ucur = unext;
+    }
+    if (fabs(dcur) < ptol) dcur = (dcur < 0.0) ? -ptol : ptol;
+    col.f(1, d - 1) = recip(dcur);
+    col.f(2, d - 1) = 0.0;
+    col.f(3, d - 1) = 0.0;
+    col.X(d - 1) = bc;
+    return apply_u(col, d);
+}
+
+// Second solve, with the first one's factors, from x of squared norm s2.
+__device__ __forceinline__ double tri_resolve(const Column& col, int d, double s2) {
+    apply_pl(col, d, 1.0 / sqrt(s2));
+    return apply_u(col, d);
+}
+
 // Eigenvectors l0 .. l1 of one cluster, unnormalised, to the columns of Sv;
 // xs[l] = ||S(:, l)||^2.  fac: 5 d^2 doubles for the LU factors.
 __device__ __forceinline__ void tri_vectors(int l0, int l1, int d, const double* dd, const double* ee,
                                             const double* lamv, double* xs, double tnorm, double* Sv, double* fac,
                                             bool& bad) {
-    const double ptol = kEps * tnorm;
     double sprev = -INFINITY;
     for (int l = l0; l <= l1; l++) {
-        double sg = lamv[l];
-        const double pert = 10.0 * kEps * fmax(fabs(sg), 1e-3 * tnorm);
-        if (l > l0 && sg <= sprev + pert) sg = sprev + pert;
+        const double sg = tri_shift(lamv[l], sprev, tnorm);
         sprev = sg;
         const Column col{Sv + l, fac + l, (size_t)d, (size_t)d * d};
-        // T - sg I = P L U with partial pivoting ([q][i]: 0 multiplier,
-        // 1 reciprocal pivot, 2-3 superdiagonals of U, 4 interchange),
-        // fused with L^{-1} P applied to the start vector
-        double dcur = dd[0] - sg, ucur = d > 1 ? ee[0] : 0.0;
-        double bc = start_value((uint32_t)l, 0u);
-        for (int i = 0; i + 1 < d; i++) {
-            const double sub = ee[i];
-            double dnext = dd[i + 1] - sg;
-            double unext = (i + 2 < d) ? ee[i + 1] : 0.0;
-            const double bn = start_value((uint32_t)l, (uint32_t)(i + 1));
-            double f, u0, u1, u2, sw, xi;
-            if (fabs(dcur) >= fabs(sub)) {
-                if (fabs(dcur) < ptol) dcur = (dcur < 0.0) ? -ptol : ptol;
-                f = sub * recip(dcur);
-                u0 = dcur;
-                u1 = ucur;
-                u2 = 0.0;
-                sw = 0.0;
-                dnext = fma(-f, ucur, dnext);
-                xi = bc;
-                bc = fma(-f, bc, bn);
-            } else {
-                f = dcur * recip(sub);
-                u0 = sub;
-                u1 = dnext;
-                u2 = unext;
-                sw = 1.0;
-                dnext = fma(-f, dnext, ucur);
-                unext = -f * unext;
-                xi = bn;
-                bc = fma(-f, bn, bc);
-            }
-            col.f(0, i) = f;
-            col.f(1, i) = recip(u0);
-            col.f(2, i) = u1;
-            col.f(3, i) = u2;
-            col.f(4, i) = sw;
-            col.X(i) = xi;
-            dcur = dnext;
-            ucur = unext;
-        }
-        if (fabs(dcur) < ptol) dcur = (dcur < 0.0) ? -ptol : ptol;
-        col.f(1, d - 1) = recip(dcur);
-        col.f(2, d - 1) = 0.0;
-        col.f(3, d - 1) = 0.0;
-        col.X(d - 1) = bc;
-        double s2 = apply_u(col, d);
+        double s2 = tri_solve(col, l, d, dd, ee, sg, tnorm);
         if (l > l0) s2 = orthogonalise(col, d, Sv, l0, l, xs);
-        apply_pl(col, d, 1.0 / sqrt(s2));
-        s2 = apply_u(col, d);
+        s2 = tri_resolve(col, d, s2);
         if (l > l0) s2 = orthogonalise(col, d, Sv, l0, l, xs);
         if (!(s2 > 0.0) || !isfinite(s2)) {
             bad = true;

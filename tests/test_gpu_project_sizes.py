@@ -11,6 +11,8 @@ within a small multiple of d eps max|l| of the exact one; eps d 100 (1.4e-12 at
 d = 64) leaves room for the eigensolver's clusters, whose vectors are
 orthogonal to about 1e-5 / gap eps.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -103,10 +105,27 @@ def _degenerate_sequence(kind, d, rng):
 
 
 @pytest.mark.parametrize("kind", ["ends", "integers", "one", "rank"])
-@pytest.mark.parametrize("dims", [[17, 31, 32, 33, 47, 48, 49, 63, 64], [65, 96, 128, 224]], ids=["to64", "to224"])
+@pytest.mark.parametrize("dims", [[17, 31, 32, 33, 47, 48, 49, 63, 64], [65, 96, 128, 224], [225, 257, 300, 417]],
+                         ids=["to64", "to224", "to417"])
 def test_projection_of_degenerate_blocks(kind, dims):
     rng = np.random.default_rng([len(dims), len(kind), 1])
     _check_sequences(kind, dims, [_degenerate_sequence(kind, d, rng) for d in dims])
+
+
+def test_cluster_of_a_large_block_is_shared():
+    """397 equal eigenvalues of 417: 80 ms with a workgroup orthogonalising their
+    vectors; one thread (some 300 000 dependent column passes) takes above ten
+    seconds."""
+    d, rng = 417, np.random.default_rng(5)
+    U = _degenerate_sequence("rank", d, rng)[2]
+    S = BPSDPSolver(d * d, 1, options(e_convergence=1e-30, r_convergence=1e-30, maxiter=10 ** 6))
+    S.set_mu(1.0)
+    for cost in (np.eye(d), -U):  # the first call also sets up
+        t0 = time.perf_counter()
+        S.solve(np.zeros(d * d), np.zeros(1), cost.ravel(), [d], 1, lambda u: np.zeros(1), lambda y: np.zeros(d * d))
+        seconds = time.perf_counter() - t0
+    S.close()
+    assert seconds < 2.0, seconds
 
 
 def _check(kind, dims):
