@@ -13,6 +13,7 @@
 #include <stdexcept>
 
 #include "refine.hpp"
+#include "refine_pair.hpp"
 
 namespace v2h {
 
@@ -129,6 +130,7 @@ __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, cons
     const bool coupled = p.epi == kEpiFinal && rs.coupled;
     const double* A = slot(R, b, coupled ? kSlotK : (p.a >= 0 ? p.a : rs.xfinal));
     const double* Bm = slot(R, b, p.b >= 0 ? p.b : rs.xfinal);
+    const double* Gm = slot(R, b, kSlotG);
     const double* sc = lam_of(R, b);
     const double mu = B.st[b.inst].mu;
     const double inv_mu = 1.0 / mu;
@@ -171,9 +173,14 @@ __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, cons
             const int gn = n0 + n, gkb = k0 + kb;
             rb[e] = (gn < d && gkb < d) ? (p.bm == kBT ? Bm[(int64_t)gn * d + gkb] : Bm[(int64_t)gkb * d + gn]) : 0.0;
             if (MIDDLE && gn < d && gkb < d) {
-                const double lk_ = sc[gkb], ln_ = sc[gn], sv = 0.5 * (rb[e] + Bm[(int64_t)gn * d + gkb]);
-                const bool near = fabs(ln_ - lk_) <= rs.om && fabs(sv) <= rs.om;
-                rb[e] = gn == gkb ? fmax(ln_, 0.0) : (near && coupling_kind(sv, lk_, ln_, rs.keep, d) == 1 ? sv : 0.0);
+                if (gn == gkb) {
+                    rb[e] = fmax(sc[gn], 0.0);
+                } else {  // as in k_ref_etile
+                    const double nk = 1.0 / sqrt(Gm[(int64_t)gkb * d + gkb]), nn = 1.0 / sqrt(Gm[(int64_t)gn * d + gn]);
+                    const RefPair pr = ref_pair(sc[gkb], sc[gn], nk, nn, Gm[(int64_t)gkb * d + gn], rb[e],
+                                                Bm[(int64_t)gn * d + gkb], rs.om);
+                    rb[e] = pr.close && coupling_kind(pr.sa, sc[gkb], sc[gn], rs.keep, d) == 1 ? pr.sa : 0.0;
+                }
             }
         }
     };
@@ -388,22 +395,20 @@ __global__ __launch_bounds__(kNT) void k_ref_etile(RefDev R, RefParams P, int k,
     for (int q = 0; q < 4; q++) {
         const int r = r0 + 8 * q, i = i0 + r;
         if (i >= d || j >= d) continue;
-        const double nn = ni_s[r] * nj_s[c], li = li_s[r], lj = lj_s[c];
+        const double li = li_s[r], lj = lj_s[c];
         double ev;
         if (i == j) {
             ev = nj_s[c] - 1.0;
             E[(int64_t)i * d + j] = ev;
         } else {
-            const double rr = -gv4[q] * nn, sv = 0.5 * (sv4[q] + tt[c][r]) * nn;
-            const double dl = lj - li, sa = fma(0.5 * (lj + li), rr, sv);
-            ev = 0.5 * rr;
-            if (fabs(dl) > om || fabs(sa) > om) {
-                const double ta = sa + sa;
-                ev += ta / (dl + copysign(sqrt(fma(dl, dl, ta * ta)), dl));
+            const RefPair pr = ref_pair(li, lj, ni_s[r], nj_s[c], gv4[q], sv4[q], tt[c][r], om);
+            ev = 0.5 * pr.rr;
+            if (!pr.close) {
+                ev += ref_rotation(pr);
             } else {
-                const int kind = coupling_kind(sv, li, lj, keep, d);
-                if (kind == 1) m[2] = fmax(m[2], fabs(sv));
-                if (kind == 2) m[1] = nmax(m[1], fabs(sv));
+                const int kind = coupling_kind(pr.sa, li, lj, keep, d);
+                if (kind == 1) m[2] = fmax(m[2], fabs(pr.sa));
+                if (kind == 2) m[1] = nmax(m[1], fabs(pr.sa));
             }
             E[(int64_t)i * d + j] = ni_s[r] * ev;
         }

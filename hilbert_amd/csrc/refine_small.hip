@@ -16,6 +16,7 @@
 #include <cmath>
 
 #include "refine.hpp"
+#include "refine_pair.hpp"
 
 namespace v2h {
 
@@ -166,24 +167,22 @@ __device__ __forceinline__ void ref_small(const BatchDev& B, const SmallDev& R, 
                     const int i = m0 + 4 * r + lk;
                     double ev = 0.0, ei = 0.0, mid = 0.0;  // correction, E, middle factor
                     if (i < d && j < d) {
-                        const double ni = nrm[i], li_ = lam[i], nn = ni * nj;
+                        const double ni = nrm[i], li_ = lam[i];
                         if (i == j) {
                             ev = ei = nj - 1.0;
                             mid = fmax(lj, 0.0);
                         } else {
-                            const double rr = -g[c][r] * nn, sv = 0.5 * (s[c][r] + UK[j * LD + i]) * nn;
-                            const double dl = lj - li_, sa = fma(0.5 * (lj + li_), rr, sv);
-                            ev = 0.5 * rr;
-                            if (fabs(dl) > om || fabs(sa) > om) {
-                                const double ta = sa + sa;
-                                ev += ta / (dl + copysign(sqrt(fma(dl, dl, ta * ta)), dl));
-                            } else if (!(fabs(sv) <= keep)) {
+                            const RefPair p = ref_pair(li_, lj, ni, nj, g[c][r], s[c][r], UK[j * LD + i], om);
+                            ev = 0.5 * p.rr;
+                            if (!p.close) {
+                                ev += ref_rotation(p);
+                            } else if (!(fabs(p.sa) <= keep)) {
                                 const double lo = fmin(lj, li_), hi = fmax(lj, li_);
-                                if (lo > DP * fabs(sv)) {
-                                    mid = sv;
-                                    mk = fmax(mk, fabs(sv));
-                                } else if (!(hi < -DP * fabs(sv))) {
-                                    mc = nmax(mc, fabs(sv));
+                                if (lo > DP * fabs(p.sa)) {
+                                    mid = p.sa;
+                                    mk = fmax(mk, fabs(p.sa));
+                                } else if (!(hi < -DP * fabs(p.sa))) {
+                                    mc = nmax(mc, fabs(p.sa));
                                 }
                             }
                             ei = ni * ev;
