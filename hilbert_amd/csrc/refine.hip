@@ -178,7 +178,7 @@ __device__ void ref_tile(const BatchDev& B, const RefDev& R, const Prod& p, cons
                 } else {  // as in k_ref_etile
                     const double nk = 1.0 / sqrt(Gm[(int64_t)gkb * d + gkb]), nn = 1.0 / sqrt(Gm[(int64_t)gn * d + gn]);
                     const RefPair pr = ref_pair(sc[gkb], sc[gn], nk, nn, Gm[(int64_t)gkb * d + gn], rb[e],
-                                                Bm[(int64_t)gn * d + gkb], rs.om);
+                                                Bm[(int64_t)gn * d + gkb], rs.om, gkb < gn);
                     rb[e] = pr.close && coupling_kind(pr.sa, sc[gkb], sc[gn], rs.keep, d) == 1 ? pr.sa : 0.0;
                 }
             }
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(kNT) void k_ref_etile(RefDev R, RefParams P, int k,
             ev = nj_s[c] - 1.0;
             E[(int64_t)i * d + j] = ev;
         } else {
-            const RefPair pr = ref_pair(li, lj, ni_s[r], nj_s[c], gv4[q], sv4[q], tt[c][r], om);
+            const RefPair pr = ref_pair(li, lj, ni_s[r], nj_s[c], gv4[q], sv4[q], tt[c][r], om, i < j);
             ev = 0.5 * pr.rr;
             if (!pr.close) {
                 ev += ref_rotation(pr);

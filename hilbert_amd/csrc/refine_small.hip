@@ -172,7 +172,7 @@ __device__ __forceinline__ void ref_small(const BatchDev& B, const SmallDev& R, 
                             ev = ei = nj - 1.0;
                             mid = fmax(lj, 0.0);
                         } else {
-                            const RefPair p = ref_pair(li_, lj, ni, nj, g[c][r], s[c][r], UK[j * LD + i], om);
+                            const RefPair p = ref_pair(li_, lj, ni, nj, g[c][r], s[c][r], UK[j * LD + i], om, i < j);
                             ev = 0.5 * p.rr;
                             if (!p.close) {
                                 ev += ref_rotation(p);
