@@ -244,7 +244,7 @@ __device__ __forceinline__ double tri_eigenvalue(int l, int d, const double* dd,
                 // neighbour of it: next to one of high multiplicity S is large and
                 // the step small, however far eigenvalue l is.  A count across
                 // s tells (bisecting instead: 33 passes per eigenvalue of a random
-                // 224-row T, against 16).
+                // 224-row T, against 15).
                 if (!probed) {
                     probed = true;
                     const double x = s <= lo ? lo + 2.0 * abstol : hi - 2.0 * abstol;
@@ -258,7 +258,14 @@ __device__ __forceinline__ double tri_eigenvalue(int l, int d, const double* dd,
                 }
             }
             newton = inside && fabs(step) <= 0.5 * last;
-            if (newton) last = fabs(step);
+            if (newton) {
+                last = fabs(step);
+                // a little past the root, so that the step there points back into
+                // the bracket whatever its rounding (with the count above alone,
+                // which every eigenvalue would take then, 16 passes instead of 15)
+                const double over = sn + copysign(abstol, step);
+                if (over > lo && over < hi) sn = over;
+            }
         }
         if (!newton) {
             sn = 0.5 * (lo + hi);
