@@ -554,15 +554,17 @@ __device__ void project_jacobi16(const BatchDev& B, const ProjItem& it, double* 
     }
     nrm = block_sum<NT>(nrm, red);
     const double thr = 1e-30 * nrm;  // (1e-15 ||A||_F)^2
-    int nsweep = 0;
-    for (; nsweep < max_sweeps; nsweep++) {
+    auto off2 = [&] {
         double off = 0.0;
         for (int e = t; e < dp * dp; e += NT) {
             const int i = e / dp, j = e - i * dp;
             if (i < j) off += 2.0 * A[pk(i, j)] * A[pk(i, j)];
         }
-        off = block_sum<NT>(off, red);
-        if (off <= thr) break;
+        return block_sum<NT>(off, red);
+    };
+    int nsweep = 0;
+    for (; nsweep < max_sweeps; nsweep++) {
+        if (off2() <= thr) break;
         for (int r = 0; r < dp - 1; r++) {
             if (t < m) {
                 int p, q;
@@ -591,7 +593,12 @@ __device__ void project_jacobi16(const BatchDev& B, const ProjItem& it, double* 
             lds_sync();
         }
     }
-    if (nsweep == max_sweeps && t == 0) atomicOr(&st.status, (int)kStatusJacobiNotConverged);
+    if (nsweep == max_sweeps) {
+        // thr is close to the rounding of a sweep, d eps ||A||, which a block with
+        // groups of equal eigenvalues can make anew in each; such a block is done
+        const double off = off2();
+        if (!(off <= 100.0 * thr) && t == 0) atomicOr(&st.status, (int)kStatusJacobiNotConverged);
+    }
 
     // x = U+ / mu, z = U+ - sym(U), v1 = c - z; partial c.x and dual residual
     double ex = 0.0, dr = 0.0;

@@ -137,8 +137,9 @@ def _degenerate_sequence(kind, d, rng):
 
 
 @pytest.mark.parametrize("kind", ["ends", "integers", "one", "rank"])
-@pytest.mark.parametrize("dims", [[17, 31, 32, 33, 47, 48, 49, 63, 64], [65, 96, 128, 224], [225, 257, 300, 417]],
-                         ids=["to64", "to224", "to417"])
+@pytest.mark.parametrize("dims", [SMALL, [13, 14, 15, 16] * 8, [17, 31, 32, 33, 47, 48, 49, 63, 64],
+                                  [65, 96, 128, 224], [225, 257, 300, 417]],
+                         ids=["small", "to16", "to64", "to224", "to417"])
 def test_projection_of_degenerate_blocks(kind, dims):
     rng = np.random.default_rng([len(dims), len(kind), 1])
     _check_sequences(kind, dims, [_degenerate_sequence(kind, d, rng) for d in dims])
