@@ -61,3 +61,17 @@ def test_traffic_lookup_reads_the_committed_summary():
     got = bench.load_traffic("cg_a", "c2v16x128")
     assert got is not None and 5e8 < got < 5e9
     assert bench.load_traffic("cg_a", "no_such_workload") is None
+
+
+def test_refinement_steps_have_one_default():
+    """A Batch starts with the steps that set_refine_params and the benchmark
+    leave it with when only something else is asked for."""
+    import inspect
+    import re
+
+    from hilbert_amd.batch import Batch
+    src = open(os.path.join(os.path.dirname(bench.__file__), "hilbert_amd", "csrc", "refine.hpp")).read()
+    steps = int(re.search(r"int max_steps = (\d+);", src).group(1))
+    assert inspect.signature(Batch.set_refine_params).parameters["max_steps"].default == steps
+    text = open(bench.__file__).read()
+    assert int(re.search(r'"--refine-steps", type=int, default=(\d+)', text).group(1)) == steps
