@@ -68,22 +68,20 @@ CONV = [5e-8, 5e-7]
 
 
 def bytes_per_instance(kind, n_p, n_d):
-    """HBM bytes of the vectors of one launch for one instance, as the plain
-    recurrences with w = A q stored have them (the count that earlier figures
-    and the traffic records use; the kernels now read r and q and write q in
-    cg_at, and read q and read and write r, p, y in cg_a: 8 (2 n_p + n_d) and
-    8 (n_p + 6 n_d))."""
-    return 8 * {"cg_at": n_p + 3 * n_d,        # write q; read r, w, p
-                "cg_a": n_p + 8 * n_d,         # read q; read+write y, r, p, w
-                "pre": 3 * n_p + 5 * n_d,      # read c-z, x, A^T y; write 3; read b, y
+    """HBM bytes of the vectors that one launch of the kernel reads and writes
+    for one instance, each once (pre: with the first residual of the CG, which
+    its timer holds)."""
+    return 8 * {"cg_at": 2 * n_p + n_d,        # read r; read+write q
+                "cg_a": n_p + 6 * n_d,         # read q; read+write y, r, p
+                "pre": 3 * n_p + 7 * n_d,      # read c-z, x, A^T y, b, y; write, then read, both pieces of r; write r
                 "post": 4 * n_p + n_d}[kind]   # read y, x, c; write A^T y, U
 
 
 # with the refinement on, the classes above 64 rows time only their fallback
-# launches, so their work per launch is an upper bound
-PROJ_CLASSES = (("project_jacobi16", 0, 16), ("project_tri64", 17, 64), ("project_tri128", 65, 128),
-                ("project_tri192", 129, 192), ("project_tri224", 193, 224), ("project_tri256", 225, 256),
-                ("project_jacobi_big", 257, 1 << 30))
+# launches, so their work per launch is an upper bound; blocks of up to 16 rows
+# are launched with those of up to 64 where there are any
+PROJ_CLASSES = (("project_jacobi16", 1, 16), ("project_tri64", 1, 64), ("project_tri128", 65, 128),
+                ("project_tri192", 129, 192), ("project_tri224", 193, 224), ("project_jacobi_big", 225, 1 << 30))
 
 
 def project_flops(dims):
@@ -133,10 +131,9 @@ def load_traffic(kernel, workload):
 
 def executions(kind, oiter, iiter):
     """Launches of `kind` that one instance takes part in, from its outer and
-    CG iteration counts: every CG solve runs one step more than it counts
-    (the step whose residual stops it)."""
+    CG iteration counts."""
     if kind in ("cg_at", "cg_a"):
-        return iiter + oiter
+        return iiter
     if kind == "pre":
         return oiter + 1
     return oiter  # post and the projection classes
@@ -151,6 +148,8 @@ def roofline(B, kt, counts, workload, dom=None, proj=None):
     launches."""
     n_p, n_d = B.n_primal, B.n_dual
     totals = {k: v[0] for k, v in kt.items() if v[1]}
+    if kt.get("cg_at", (0, 0))[1] != kt.get("cg_a", (0, 0))[1]:
+        totals.pop("cg_at", None)  # its timer also holds whole CG solves (SDPs that fit one workgroup)
     if dom is None:
         dom = max(totals, key=totals.get)
     ms, cnt = kt[dom]

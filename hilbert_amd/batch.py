@@ -344,7 +344,8 @@ class Batch:
 
     def kernel_times(self, full=False) -> dict:
         """{kind: (total ms, launches)}; full=True: only launches that
-        processed the whole batch (every instance running)."""
+        processed the whole batch (every instance running).  SDPs whose CG
+        fits one workgroup have all its steps in one launch, under "cg_at"."""
         n = len(self.KERNEL_KINDS)
         ms = np.zeros(n)
         cnt = np.zeros(n, dtype=np.int64)

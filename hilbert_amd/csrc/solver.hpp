@@ -188,7 +188,7 @@ class Batch {
     hipStream_t stream() const { return stream_; }
 
     // HIP-event timing of every kernel launch of solve(), per kernel kind:
-    // 0 pre, 1 cg_at, 2 cg_a, 3 post, 4..10 projection classes: d <= 16 (timed
+    // 0 pre, 1 cg_at and (whole CG solves) cg_small, 2 cg_a, 3 post, 4..10 projection classes: d <= 16 (timed
     // with the next where a batch has both), d <= 64 with its refinement, the
     // tridiagonal eigensolver of d <= 128 / 192 / 224, (unused), d > 224; 11: the device part of one set_df_integrals (its
     // contraction kernels and the cost packing); 12: the pair Gram matrix of

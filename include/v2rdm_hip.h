@@ -271,7 +271,9 @@ int v2h_batch_Au_noalloc(v2h_batch *b, int inst, const double *u, double *out);
 
 /* HIP-event timing of the kernels launched by v2h_batch_solve, recorded on
  * the library's stream.  ms[16] and counts[16] per kernel kind: 0 iteration
- * start (A [c - z, x, A^T y]), 1 CG A^T p, 2 CG A q, 3 A^T y and U, 4..10 PSD
+ * start (A [c - z, x, A^T y] and the CG's first residual), 1 CG A^T p, 2 CG A q
+ * (the CG of the SDPs that fit one workgroup is one launch of all its steps,
+ * under 1; with such SDPs the counts of 1 and 2 differ), 3 A^T y and U, 4..10 PSD
  * projection classes by rows: up to 16 (launched with the next), up to
  * 64 / 128 / 192 / 224, up to 256 (launched with the next), above 224;
  * 11 the device part of v2h_batch_set_df_integrals (from the first

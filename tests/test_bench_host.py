@@ -22,13 +22,13 @@ class _FakeBatch:
 def test_cg_a_roofline_by_hand():
     B = _FakeBatch([100, 120], [200, 240], [[4], [4]])
     counts = [(10, 90), (20, 180)]  # (outer, CG) iterations of each instance
-    # cg_a launches an instance takes part in: CG steps + one per outer iteration
-    runs = [90 + 10, 180 + 20]
-    launches = 200                  # the kernel's launches (the longer instance's)
+    # cg_a launches an instance takes part in: its CG steps
+    runs = [90, 180]
+    launches = 200                  # the kernel's launches (those of the longer instance and a margin)
     kt = {"cg_a": (2.0, launches), "cg_at": (1.0, launches), "post": (0.5, 20)}
     dom, r = bench.roofline(B, kt, counts, "no_such_workload")
     assert dom == "cg_a"
-    work = (runs[0] * 8 * (100 + 8 * 200) + runs[1] * 8 * (120 + 8 * 240)) / launches
+    work = (runs[0] * 8 * (100 + 6 * 200) + runs[1] * 8 * (120 + 6 * 240)) / launches
     assert r["work_per_launch"] == pytest.approx(work)
     assert r["per_launch_ms"] == pytest.approx(2.0 / launches)
     assert r["achieved"] == pytest.approx(work / (2.0 / launches * 1e-3) / 1e9)
@@ -41,9 +41,18 @@ def test_named_kernel_and_bytes_per_instance():
     kt = {"cg_a": (2.0, 10), "cg_at": (1.0, 10)}
     dom, r = bench.roofline(B, kt, [(1, 9)], "none", "cg_at")
     assert dom == "cg_at"
-    assert r["work_per_launch"] == pytest.approx(10 * 8 * (100 + 3 * 200) / 10)
+    assert r["work_per_launch"] == pytest.approx(9 * 8 * (2 * 100 + 200) / 10)
     assert bench.bytes_per_instance("post", 10, 3) == 8 * (4 * 10 + 3)
     assert bench.executions("pre", 5, 40) == 6 and bench.executions("post", 5, 40) == 5
+
+
+def test_whole_cg_solves_stay_out_of_the_gather_roofline():
+    """SDPs whose CG is one launch are timed as cg_at without a cg_a."""
+    B = _FakeBatch([100], [200], [[4]])
+    dom, _ = bench.roofline(B, {"cg_at": (9.0, 30), "cg_a": (2.0, 20), "post": (1.0, 10)}, [(10, 20)], "none")
+    assert dom == "cg_a"
+    dom, _ = bench.roofline(B, {"cg_at": (9.0, 10), "post": (1.0, 10)}, [(10, 20)], "none")
+    assert dom == "post"
 
 
 def test_refinement_roofline_from_device_flops():
