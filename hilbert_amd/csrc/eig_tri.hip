@@ -583,7 +583,7 @@ __device__ void project_jacobi16(const BatchDev& B, const ProjItem& it, double* 
                 rs[t] = s;
             }
             lds_sync();
-            apply_round<NT>(A, pp, qq, rc, rs, m, 1.0, true);
+            apply_round<NT>(A, pp, qq, rc, rs, m);
             for (int e = t; e < m * dp; e += NT) {  // columns p, q of V
                 const int k = e / dp, i = e - k * dp;
                 const double c = rc[k], s = rs[k], vp = V[i][pp[k]], vq = V[i][qq[k]];

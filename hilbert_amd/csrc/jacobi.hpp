@@ -36,39 +36,28 @@ __device__ __forceinline__ void tri_pair(int e, int& P, int& Q) {
     P = e - qq * (qq + 1) / 2;
 }
 
-// One round of two-sided rotations on the packed matrix A.  sgn = +1 applies
-// G_P T G_Q^T (forward), sgn = -1 applies G_P^T T G_Q (replay).  In the
-// forward direction the 2x2 diagonal tiles are set to their closed form.
+// One round of two-sided rotations G_P A G_Q^T on the packed matrix A; the 2x2
+// diagonal tiles are set to their closed form.
 template <int NT>
-__device__ void apply_round(double* A, const int* pp, const int* qq, const double* rc, const double* rs,
-                            int m, double sgn, bool forward) {
+__device__ void apply_round(double* A, const int* pp, const int* qq, const double* rc, const double* rs, int m) {
     const int ntile = m * (m + 1) / 2;
     for (int e = threadIdx.x; e < ntile; e += NT) {
         int P, Q;
         tri_pair(e, P, Q);
-        const double cP = rc[P], sP = sgn * rs[P];
+        const double cP = rc[P], sP = rs[P];
         const int p = pp[P], q = qq[P];
         if (P == Q) {
             const int ipp = pk(p, p), ipq = pk(p, q), iqq = pk(q, q);
-            double app = A[ipp], apq = A[ipq], aqq = A[iqq];
-            if (forward) {
-                if (rs[P] != 0.0) {
-                    double t = rs[P] / rc[P];
-                    A[ipp] = app - t * apq;
-                    A[iqq] = aqq + t * apq;
-                    A[ipq] = 0.0;
-                }
-            } else {
-                // T = G^T T' G with G = [[c, -s], [s, c]] (s already negated by sgn)
-                double r00 = cP * app - sP * apq, r01 = cP * apq - sP * aqq;
-                double r10 = sP * app + cP * apq, r11 = sP * apq + cP * aqq;
-                A[ipp] = cP * r00 - sP * r01;
-                A[ipq] = sP * r00 + cP * r01;
-                A[iqq] = sP * r10 + cP * r11;
+            const double app = A[ipp], apq = A[ipq], aqq = A[iqq];
+            if (rs[P] != 0.0) {
+                const double t = rs[P] / rc[P];
+                A[ipp] = app - t * apq;
+                A[iqq] = aqq + t * apq;
+                A[ipq] = 0.0;
             }
             continue;
         }
-        const double cQ = rc[Q], sQ = sgn * rs[Q];
+        const double cQ = rc[Q], sQ = rs[Q];
         const int r = pp[Q], s = qq[Q];
         const int i0 = pk(p, r), i1 = pk(p, s), i2 = pk(q, r), i3 = pk(q, s);
         double a0 = A[i0], a1 = A[i1], a2 = A[i2], a3 = A[i3];

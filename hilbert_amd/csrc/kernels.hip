@@ -765,7 +765,6 @@ __global__ void k_cost_adjoint(const int32_t* ptr, const int32_t* ent, const dou
     }
 }
 
-// out[0] = sum_i a[i] b[i] in one workgroup (fixed order)
 // a . b in two launches with a fixed summation order: kDotParts workgroups
 // each reduce one contiguous chunk into out[1 + part], then one workgroup
 // sums the parts in order into out[0].

@@ -14,7 +14,7 @@
 // (the second term is their a_ij / (l_j - l_i) for small a_ij, limited like a
 // Jacobi rotation), which converges quadratically, restores the orthogonality
 // of X in the same step, and then U+ = X diag(l+) X^T.  Pairs inside a cluster
-// threshold keep only r_ij / 2 and their coupling beside diag(l+).  A block
+// threshold keep only r_ij / 2 and, beside diag(l+), their coupling a_ij.  A block
 // whose correction does not fall below the acceptance threshold within
 // max_steps steps, and every block without eigenvectors yet (first iteration,
 // after a reset), takes a tridiagonal eigensolver instead (eig_tri.hip, above
@@ -123,7 +123,7 @@ constexpr int kMaxSteps = 8;
 void launch_ref_state(const BatchDev& B, const RefDev& R, hipStream_t s);
 // sym(U) of the refining blocks.
 void launch_ref_sym(const BatchDev& B, const RefDev& R, hipStream_t s);
-// One refinement step k (1..3): X_in = V (k = 1), Xa (k = 2), Xb (k = 3).
+// One refinement step k (1..max_steps): X_in = V (k = 1), then Xa and Xb in turn.
 void launch_ref_step(const BatchDev& B, const RefDev& R, const RefParams& P, int k, hipStream_t s);
 // x = X diag(l+) X^T / mu with z, v1, partial sums; the block's projection sums.
 void launch_ref_final(const BatchDev& B, const RefDev& R, hipStream_t s);

@@ -3,10 +3,13 @@
 // Per outer iteration (all instances of the batch at once, converged ones
 // skipped inside the kernels):
 //   k_pre      A [c - z, x, A^T y]; finish the previous iteration
-//   CG steps   (k_cg_at, k_cg_a) until every instance's CG has stopped
+//   CG         k_cg_at and k_cg_a steps until every instance's CG has stopped;
+//              k_cg_small for the SDPs whose CG fits one workgroup
 //   k_post     A^T y, U = mu x + A^T y - c
-//   k_project  one workgroup per PSD block (four size classes)
-// The host only reads the small per-instance state array between CG chunks.
+//   projection refinement and eigensolvers by size class (projector.hpp)
+// The host reads the small per-instance state array between CG chunks (where
+// every SDP is small, after some iterations), and which blocks above 224 rows
+// need their eigensolver.
 #include "solver.hpp"
 
 #include <algorithm>

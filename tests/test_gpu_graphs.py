@@ -1,7 +1,7 @@
 """GPU: hipGraph replay of the outer iteration's first CG chunk.
 
 Mode GRAPHS_CG captures the first CG chunk of every outer iteration (its
-k_cg_at / k_cg_a / k_cg_reduce launches) once per launch plan and step count
+k_cg_at / k_cg_a launches) once per launch plan and step count
 and replays it (with the kernel timers off; with them on the launches go one
 by one); GRAPHS_ALL also captures k_post and the whole projection, with the
 eigenvector formation as a branch of the next CG graph.  Without graphs

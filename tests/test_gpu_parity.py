@@ -244,12 +244,12 @@ def _eigh_projection(U, dims):
 
 PROJ_CASES = {
     # blocks: Hubbard 8 (128, 64, 28, 8), C1 n=10 (200, 100, 45, 10),
-    # (16e,16o) C2v (up to about 180), C1 n=11 (242: matrix in global memory)
+    # (16e,16o) C2v (up to about 180), C1 n=11 (242: reduced by the whole GPU)
     "hubbard8": lambda: (Problem(8, 4, 4), *hubbard_integrals(8, 1.0, 4.0)),
     "c1_10": lambda: _synthetic(10, 30, 1, 11),
     "c2v_16": lambda: _synthetic(16, 48, 4, 12),
     "c1_11": lambda: _synthetic(11, 20, 1, 13),
-    # C1 n=12 (G2aa 288: Jacobi in global memory); first instance of the
+    # C1 n=12 (G2aa 288); first instance of the
     # large D2h batch, (20e,20o)-(24e,24o) (blocks up to about 180)
     "c1_12": lambda: _synthetic(12, 20, 1, 14),
     "batch16_big_0": lambda: __import__("hilbert_amd.configs", fromlist=["x"]).batch16_big(1)[0],

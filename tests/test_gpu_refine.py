@@ -1,9 +1,9 @@
-"""GPU: the warm-started projection of the PSD blocks of 65..256 rows.
+"""GPU: the warm-started projection of the PSD blocks above 64 rows.
 
 Each outer iteration refines the previous iteration's eigenvectors with FP64
 matrix-core products (Ogita-Aishima iterative refinement) and falls back to
-the tridiagonal eigensolver for blocks without eigenvectors or whose
-refinement is not accepted.  Checked here: x = U+ / mu against LAPACK (numpy
+an eigensolver for blocks without eigenvectors or whose refinement is not
+accepted.  Checked here: x = U+ / mu against LAPACK (numpy
 eigh) on iterations that take the refined path, the refined path actually
 taken once U changes slowly, the solve's optimum equal to the one with the
 tridiagonal eigensolver alone, and a batch equal to its instances solved
@@ -74,7 +74,7 @@ def test_refined_projection_matches_eigh(name):
     s1 = B.projection_stats()
     refined = s1["refined"] - s0["refined"]
     fallback = s1["fallback"] - s0["fallback"]
-    print(f"{name}: {nref} blocks of 65..256, 3 iterations: {refined} refined, {fallback} fallback; "
+    print(f"{name}: {nref} blocks above 64 rows, 3 iterations: {refined} refined, {fallback} fallback; "
           f"whole run {s1}", flush=True)
     assert refined + fallback == 3 * nref
     if name != "hubbard8":
