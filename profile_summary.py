@@ -126,9 +126,14 @@ def counters(args):
 def traffic(args):
     fetch = read_counter(args.fetch, "FETCH_SIZE")
     write = read_counter(args.write, "WRITE_SIZE")
-    mean = lambda v: sum(v) / max(len(v), 1)
-    kf = {short_name(k): mean(v) * 1024.0 for k, v in fetch.items()}
-    kw = {short_name(k): mean(v) * 1024.0 for k, v in write.items()}
+
+    def means(values):  # bytes per dispatch; the instantiations of a template together
+        per = defaultdict(list)
+        for k, v in values.items():
+            per[short_name(k)] += v
+        return {k: 1024.0 * sum(v) / max(len(v), 1) for k, v in per.items()}
+
+    kf, kw = means(fetch), means(write)
     copy_bytes = args.copy_mib * float(1 << 20)
     cfk = max((max(v) for k, v in fetch.items() if short_name(k) == "k_copy"), default=0.0) * 1024.0
     cwk = max((max(v) for k, v in write.items() if short_name(k) == "k_copy"), default=0.0) * 1024.0
@@ -144,7 +149,7 @@ def traffic(args):
     print(f"{'kernel':24s} {'dispatches':>10s} {'fetch MB':>10s} {'write MB':>10s} {'bytes/launch':>14s}")
     for k in sorted(set(kf) | set(kw)):
         f, w = kf.get(k, 0.0) * cf, kw.get(k, 0.0) * cw
-        n = max(len(v) for kk, v in fetch.items() if short_name(kk) == k) if k in kf else 0
+        n = sum(len(v) for kk, v in fetch.items() if short_name(kk) == k)
         rec[k] = {"fetch_bytes": f, "write_bytes": w, "bytes_per_launch": f + w,
                   "fetch_factor": cf, "write_factor": cw}
         print(f"{k:24s} {n:10d} {f / 1e6:10.2f} {w / 1e6:10.2f} {f + w:14.4g}")

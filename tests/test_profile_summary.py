@@ -65,6 +65,16 @@ def test_traffic_applies_the_copy_calibration(tmp_path):
     assert data["wl"]["k_copy"]["bytes_per_launch"] == pytest.approx(2 * mib * (1 << 20))
 
 
+def test_traffic_takes_the_instantiations_of_a_kernel_together(tmp_path):
+    fetch, write = str(tmp_path / "f"), str(tmp_path / "w")
+    for d, counter in ((fetch, "FETCH_SIZE"), (write, "WRITE_SIZE")):
+        _counter_csv(d, counter, [(1, "k_copy(x)", 2048.0), (2, "void k_ref_gemm<false>(x)", 300.0),
+                                  (3, "void k_ref_gemm<false>(x)", 500.0), (4, "void k_ref_gemm<true>(x)", 1.0)])
+    out = str(tmp_path / "t.json")
+    ps.traffic(argparse.Namespace(fetch=fetch, write=write, copy_mib=2, workload="wl", out=out))
+    assert json.load(open(out))["wl"]["k_ref_gemm"]["fetch_bytes"] == pytest.approx(1024.0 * 801.0 / 3.0)
+
+
 def test_traffic_needs_the_calibration_copy(tmp_path):
     fetch, write = str(tmp_path / "f"), str(tmp_path / "w")
     _counter_csv(fetch, "FETCH_SIZE", [(1, "k_cg_a(x)", 100.0)])
