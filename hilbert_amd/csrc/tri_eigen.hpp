@@ -262,8 +262,9 @@ __device__ __forceinline__ double tri_eigenvalue(int l, int d, const double* dd,
                 last = fabs(step);
                 // a little past the root, so that the step there points back into
                 // the bracket whatever its rounding (with the count above alone,
-                // which every eigenvalue would take then, 16 passes instead of 15)
-                const double over = sn + copysign(abstol, step);
+                // which every eigenvalue would take then, 16 passes instead of 15):
+                // by more than the counts round, by less than is accepted
+                const double over = sn + copysign(1.5 * abstol, step);
                 if (over > lo && over < hi) sn = over;
             }
         }
